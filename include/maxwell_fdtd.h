@@ -314,6 +314,25 @@ typedef struct mw_program {
  * (fdtd/runtime/stepping.py:2289-2357, :1818-2024). */
 int mw_run_steps(const mw_program* program, int32_t first, int32_t count, void* stream);
 
+/* Optional buffers of a program that let several steps share one pass over the
+ * grid.  Nothing in them outlives a call (`stage` apart, whose rows are zero between
+ * calls where it matters): they need no initialisation, and a program's state after a call is where mw_run_steps leaves it.  Two calls that
+ * overlap must not share one.  No reference counterpart. */
+typedef struct mw_workspace {
+  float* psi_e_alt[6];  /* same sizes as cpml.psi[0..5] (NULL: no two-step pass with CPML) */
+  float* line_history;  /* 4 * aux.n_e floats (NULL: programs with an auxiliary line step singly) */
+  int32_t term_steps;   /* steps each SHIFTED term's `values` holds one after another (1 or 2) */
+  int32_t stage_depth;  /* rows of `stage`, a multiple of 4 up to 64 */
+  float* stage;         /* zeroed: a row per step of the samples of all observed planes and points, added to
+                           the sums a block of rows at a time; may be plane_stage where the depths agree
+                           (NULL: programs with observers step singly) */
+  int64_t stage_floats;
+} mw_workspace;
+
+/* mw_run_steps with a workspace (NULL: exactly mw_run_steps). */
+int mw_run_steps_ws(const mw_program* program, const mw_workspace* workspace, int32_t first, int32_t count,
+                    void* stream);
+
 /* ---- adjoint (reverse-mode) ----
  * Design window: the node box [lo, hi) over which dL/d(decay_E) and dL/d(curl_E)
  * are accumulated, each as three z-fastest (hi-lo) boxes, one per E component.

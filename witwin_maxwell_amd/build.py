@@ -18,7 +18,7 @@ CSRC = os.path.join(PKG, "csrc")
 LIBDIR = os.path.join(PKG, "_lib")
 LIBNAME = "libmaxwell_fdtd.so"
 SOURCES = ["maxwell_fdtd.hip"]
-HEADERS = ["yee.h", "terms.h", "fused.h", "shell.h", "zedge.h", "adjoint.h", "batch.h"]
+HEADERS = ["yee.h", "terms.h", "fused.h", "shell.h", "zedge.h", "march.h", "adjoint.h", "batch.h"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -26,7 +26,8 @@ HIPCC_FLAGS = [
     "-std=c++17",
     "-fPIC",
     "-shared",
-    "-ffp-contract=fast",
+    # fused multiply-adds wherever they fit, except where the source says otherwise
+    "-ffp-contract=fast-honor-pragmas",
     # keep packed-FP32 (v_pk_*_f32) instructions out of the device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-munsafe-fp-atomics",

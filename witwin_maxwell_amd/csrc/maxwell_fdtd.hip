@@ -17,6 +17,14 @@
 #include "terms.h"
 #include "zedge.h"
 #include "yee.h"
+// The tile march (march.h) exchanges values across a block's wavefronts; a host
+// build without block-wide lockstep leaves it out and takes the separate launches.
+#if defined(__HIP__) || defined(MW_EMULATED_BLOCKS)
+#include "march.h"
+#define MW_MARCH 1
+#else
+#define MW_MARCH 0
+#endif
 
 namespace {
 
@@ -692,6 +700,294 @@ int launch_fused(const mw_program* p, int n, hipStream_t s, mw_fields* out_field
   return MW_OK;
 }
 
+// A step's stage row: one plane per distinct (component, axis, column) of the
+// observed planes, one after another.
+struct StagePlane {
+  int component, axis, index;
+  int64_t off, cells;
+};
+struct StageLayout {
+  StagePlane planes[MW_MAX_PLANES];
+  int count = 0;
+  int64_t row_floats = 0, cells = 0;  // a row's samples, the largest plane's
+  int64_t point_off = 0;              // where the points' samples start
+  // the place of plane `o` in the row, added to it unless it is there
+  int64_t add(const mw_grid* g, const mw_plane_obs& o) {
+    for (int i = 0; i < count; ++i)
+      if (planes[i].component == o.component && planes[i].axis == o.axis && planes[i].index == o.index)
+        return planes[i].off;
+    int shp[3];
+    component_shape(g, o.component, shp);
+    const int64_t n = (int64_t)shp[0] * shp[1] * shp[2] / shp[o.axis];
+    planes[count++] = StagePlane{o.component, o.axis, o.index, row_floats, n};
+    row_floats += n;
+    cells = std::max(cells, n);
+    return row_floats - n;
+  }
+};
+
+#if MW_MARCH
+// The march's blocks.  A block's plane takes as long as its wavefronts' loads and
+// stores (about 28 cycles of a CU each, whatever they carry: 15 of them a plane for
+// fields and coefficients cost 2.8 us on a full chip at 129^3, 23 with one axis of
+// CPML or with four observed components 4.3-4.6), so tiles are weighed by their count:
+// z tiles by what lies in them, tile rows at the y ends by their layers, planes at the
+// x ends by theirs.  One block fills a CU, so the grid is cut until every CU has one:
+// the most costly block decides, and costlier tiles get more and shorter chunks.
+// Small grids, where a plane takes its latency whatever lies in it, get equal blocks
+// (73^3 with CPML and two flux planes: 32 us a step, 39 by weight; 105^3 49 and 44).
+// Layered scenes beyond four rounds of blocks of sixteen planes (two with z planes) use
+// those: many short blocks even the load out by themselves, and keep the planes in use
+// contiguous (281^3 with CPML: 395 us a step, 478 with one round of equal blocks; 185^3
+// 161, and 146 by weight; with z planes 178 and 185).
+void march_blocks(const mw_program* p, int steps, mw::MarchArgs* out) {
+  mw::MarchArgs& a = *out;
+  const mw_grid& g = p->grid;
+  const int own_z = mw::kMarchCols - 2 * steps, own_y = mw::kMarchRows - 2 * steps, halo = 2 * steps;
+  a.tiles_z = std::max(1, (g.nz - halo + own_z - 1) / own_z);
+  a.tiles_y = std::max(1, (g.ny - halo + own_y - 1) / own_y);
+  const mw_cpml& c = p->cpml;
+  auto low = [&](int axis) { return c.enabled ? std::max(c.psi_low[axis == 0 ? 2 : axis - 1], c.psi_low[axis == 0 ? 8 : axis + 5]) : 0; };
+  auto high = [&](int axis, int n) {
+    const int e = axis == 0 ? 2 : axis - 1, h = axis == 0 ? 8 : axis + 5;
+    if (!c.enabled) return n;
+    return std::min({n, c.psi_high_len[e] > 0 ? c.psi_high_start[e] : n, c.psi_high_len[h] > 0 ? c.psi_high_start[h] : n});
+  };
+  const int kPlain = 15 + 12 * a.nf_dft, kLayer = 8;
+  const int x_low = std::min(low(0), g.nx), x_high = std::max(high(0, g.nx), x_low), layers = x_low + g.nx - x_high;
+  const int tiles = a.tiles_z * a.tiles_y, extra = steps == 2 ? 4 : 1;
+  auto even = [&](int chunk) {
+    a.chunk = std::min({chunk, g.nx, mw::kMarchPlanes});
+    a.blocks = tiles * ((g.nx + a.chunk - 1) / a.chunk);
+  };
+  if (p->xchunk > 0) return even(p->xchunk);
+  bool z_planes = false;
+  for (int q = 0; q < a.n_planes; ++q) z_planes = z_planes || a.planes[q].axis == 2;
+  if (c.enabled && (int64_t)tiles * g.nx >= (z_planes ? 512 : 1024) * 16) return even(16);
+  // a tile's cost per plane
+  auto tile_cost = [&](int z) {
+    const int k0 = z * own_z, k1 = std::min(g.nz, k0 + mw::kMarchCols);
+    int cost = kPlain + (k0 < low(2) || k1 > high(2, g.nz) ? kLayer : 0);
+    for (int q = 0; q < a.n_planes; ++q)
+      if (a.planes[q].axis == 2 && a.planes[q].index >= k0 && a.planes[q].index < k1) cost += steps;
+    for (int f = 0; f < 2; ++f)
+      for (int i = 0; i < (f ? p->n_e_terms : p->n_h_terms); ++i) {
+        const mw_term& t = f ? p->e_terms[i] : p->h_terms[i];
+        if (t.offset[2] < k1 && t.offset[2] + t.shape[2] > k0 && 2 * t.shape[1] > g.ny) cost += steps;
+      }
+    return cost;
+  };
+  auto row_cost = [&](int y) {
+    return y * own_y < low(1) || std::min(g.ny, y * own_y + mw::kMarchRows) > high(1, g.ny) ? kLayer : 0;
+  };
+  int cost_z[mw::kMarchBlocks], cost_y[mw::kMarchBlocks];
+  bool alike = (int64_t)tiles * g.nx < 1536;
+  if (tiles <= mw::kMarchBlocks) {
+    bool same = layers == 0;
+    for (int z = 0; z < a.tiles_z; ++z) cost_z[z] = tile_cost(z);
+    for (int y = 0; y < a.tiles_y; ++y) cost_y[y] = row_cost(y);
+    for (int z = 1; z < a.tiles_z; ++z) same = same && cost_z[z] == cost_z[0];
+    for (int y = 1; y < a.tiles_y; ++y) same = same && cost_y[y] == cost_y[0];
+    alike = alike || same;
+  }
+  // chunks of a tile for blocks of at most `most`
+  auto chunks = [&](int z, int y, int most) {
+    const int plane = cost_z[z] + cost_y[y], all = g.nx * plane + layers * kLayer, room = most - extra * plane;
+    return std::min(g.nx, std::max((2 * g.nx + mw::kMarchPlanes - 1) / mw::kMarchPlanes,
+                                   room > 0 ? (all + room - 1) / room : g.nx));
+  };
+  auto total = [&](int most) {
+    int n = 0;
+    for (int z = 0; z < a.tiles_z; ++z)
+      for (int y = 0; y < a.tiles_y; ++y) n += chunks(z, y, most);
+    return n;
+  };
+  int lo = 0, hi = (g.nx + extra) * (kPlain + 64) + layers * kLayer + 64 * MW_MAX_TERMS;
+  if (alike || tiles > mw::kMarchBlocks || g.nx > 65535 || total(hi) > mw::kMarchBlocks) {  // whole rounds of equal blocks
+    int best = std::min(g.nx, mw::kMarchPlanes);
+    int64_t cost = INT64_MAX;
+    for (int n = (g.nx + mw::kMarchPlanes - 1) / mw::kMarchPlanes; n <= g.nx; ++n) {
+      const int chunk = (g.nx + n - 1) / n;
+      const int64_t per_xcd = ((int64_t)tiles * ((g.nx + chunk - 1) / chunk) + 7) / 8;
+      const int64_t t = ((per_xcd + 31) / 32) * (chunk + extra);
+      if (t < cost) {
+        cost = t;
+        best = chunk;
+      }
+    }
+    return even(best);
+  }
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    (total(mid) <= mw::kMarchBlocks ? hi : lo) = mid;
+  }
+  a.chunk = 0;
+  a.blocks = 0;
+  for (int y = 0; y < a.tiles_y; ++y)
+    for (int z = 0; z < a.tiles_z; ++z) {
+      const int n = chunks(z, y, hi), plane = cost_z[z] + cost_y[y], all = g.nx * plane + layers * kLayer;
+      int x = 0;
+      int64_t spent = 0;
+      for (int q = 0; q < n && x < g.nx; ++q) {
+        const int x0 = x;
+        for (; x < g.nx && (x == x0 || spent * n < (int64_t)all * (q + 1)); ++x)
+          spent += plane + (x < x_low || x >= x_high ? kLayer : 0);
+        if (q == n - 1) x = g.nx;
+        a.list[a.blocks++] = mw::MarchBlock{(uint16_t)x0, (uint16_t)x, (uint8_t)y, (uint8_t)z};
+      }
+    }
+  std::sort(a.list, a.list + a.blocks, [](const mw::MarchBlock& l, const mw::MarchBlock& r) {
+    const int dl = l.x0 + l.x1, dr = r.x0 + r.x1;
+    return dl != dr ? dl < dr : l.y != r.y ? l.y < r.y : l.z < r.z;
+  });
+}
+
+// May the program's steps be taken by the march, one at a time (1) or two (2), or
+// not at all (0)?  Explicit z tilings ask for the separate launches; periodic faces
+// need H from across the seam, which only their shell pass reads.
+int march_steps(const mw_program* p, const mw_workspace* ws, const StageLayout& stage) {
+  if (!ws || !p->fused || p->z_tiling != 0 || p->n_points > mw::kMarchPoints) return 0;
+  if (grid_periodic(p->grid)) return 0;
+  if (p->has_ade && p->ade.count[0] + p->ade.count[1] + p->ade.count[2] > 0) return 0;
+  // every observed plane and point is staged
+  if (stage.row_floats > 0 &&
+      (!ws->stage || ws->stage_depth < 4 || ws->stage_depth % 4 != 0 || ws->stage_depth > mw::kMaxStageDepth ||
+       stage.row_floats >= (1 << 30) || ws->stage_depth * stage.row_floats > ws->stage_floats))
+    return 0;
+  // z planes in a CPML scene of medium size: every block of a z tile waits for the
+  // wavefronts that store samples, and the blocks are too few to even it out (137^3 with
+  // two flux planes: 83 us a step, 75 by the separate launches; 105^3 44 against 48,
+  // 185^3 178 against 179)
+  if (p->cpml.enabled) {
+    const int64_t tiles = (int64_t)((p->grid.nz + 55) / 60) * ((p->grid.ny + 7) / 12) * p->grid.nx;
+    for (int q = 0; q < stage.count && tiles >= 4096 && tiles < 8192; ++q)
+      if (stage.planes[q].axis == 2) return 0;
+  }
+  // byte offsets within a component (two planes past its end included) are 32-bit
+  if (((int64_t)p->grid.nx + 3) * p->grid.ny * p->grid.nz * 4 >= (int64_t(1) << 32)) return 0;
+  if (p->cpml.enabled) {  // the march keeps one slab layout per family and axis
+    static const int pair[6][2] = {{0, 5}, {1, 3}, {2, 4}, {6, 11}, {7, 9}, {8, 10}};
+    for (const auto& q : pair)
+      if (p->cpml.psi_low[q[0]] != p->cpml.psi_low[q[1]] ||
+          p->cpml.psi_high_start[q[0]] != p->cpml.psi_high_start[q[1]] ||
+          p->cpml.psi_high_len[q[0]] != p->cpml.psi_high_len[q[1]])
+        return 0;
+  }
+  bool shifted = false;
+  for (int f = 0; f < 2; ++f) {
+    const mw_term* t = f ? p->e_terms : p->h_terms;
+    for (int i = 0; i < (f ? p->n_e_terms : p->n_h_terms); ++i) {
+      shifted = shifted || t[i].kind == MW_TERM_SHIFTED;
+      // a line term must sample the program's own line, whose history stands in for it
+      if (t[i].kind == MW_TERM_LINE &&
+          (!ws->line_history || p->aux.n_e <= 0 || t[i].line != (f ? p->aux.h : p->aux.e) ||
+           t[i].line_len > p->aux.n_e - f))
+        return 0;
+    }
+  }
+  if (p->aux.n_e > 0 && !ws->line_history) return 0;
+  if (shifted && ws->term_steps < 2) return 1;
+  if (p->cpml.enabled)
+    for (int q = 0; q < 6; ++q)
+      if (p->cpml.psi_low[q] + p->cpml.psi_high_len[q] > 0 && !ws->psi_e_alt[q]) return 1;
+  return 2;
+}
+
+// Arguments of a march of `steps` steps that start at an even (odd = false) or odd
+// step, reading the state where that step's state lives; `back`: reading the other
+// buffers instead and writing these (the second of two two-step marches).
+void build_march_args(const mw_program* p, const mw_workspace* ws, int steps, bool odd, bool back,
+                      const StageLayout& stage, mw::MarchArgs* out) {
+  mw::MarchArgs& a = *out;
+  memset(&a, 0, sizeof(a));
+  a.g = p->grid;
+  a.cf = p->coeffs;
+  a.cp = p->cpml;
+  const bool alt = odd != back;
+  a.in = alt ? p->fields_alt : p->fields;
+  a.out = alt ? p->fields : p->fields_alt;
+  if (p->cpml.enabled) {
+    for (int q = 0; q < 6; ++q) {
+      float* e0 = p->cpml.psi[q];
+      float* e1 = steps == 2 ? ws->psi_e_alt[q] : e0;
+      a.cp.psi[q] = back ? e1 : e0;
+      a.psi_out[q] = back ? e0 : e1;
+      a.cp.psi[6 + q] = alt ? p->psi_h_alt[q] : p->cpml.psi[6 + q];
+      a.psi_out[6 + q] = alt ? p->cpml.psi[6 + q] : p->psi_h_alt[q];
+    }
+  }
+  a.h_terms = p->h_terms_dev;
+  a.e_terms = p->e_terms_dev;
+  a.n_h_terms = p->n_h_terms;
+  a.n_e_terms = p->n_e_terms;
+  a.line_history = ws->line_history;
+  a.line_n = p->aux.n_e;
+  a.nf_dft = p->nf_dft;
+  a.dft_cos = p->dft_cos;
+  a.dft_sin = p->dft_sin;
+  for (int c = 0; c < 3; ++c) { a.dft_re[c] = p->dft_re[c]; a.dft_im[c] = p->dft_im[c]; }
+  a.n_points = p->n_points;
+  a.point_component = p->point_component;
+  a.point_linear = p->point_linear;
+  a.point_off = (int32_t)stage.point_off;
+  for (int i = 0; i < stage.count; ++i)
+    a.planes[a.n_planes++] = mw::MarchPlane{stage.planes[i].component, stage.planes[i].axis, stage.planes[i].index,
+                                            (int)stage.planes[i].off};
+  march_blocks(p, steps, &a);
+  for (int c = 0; c < 3; ++c) {
+    int se[3], sh[3];
+    component_shape(&p->grid, c, se);
+    component_shape(&p->grid, 3 + c, sh);
+    const intptr_t pe = (intptr_t)4 * se[1] * se[2], ph = (intptr_t)4 * sh[1] * sh[2];  // bytes of a plane
+    const int be = steps == 2 ? 2 : 0, bh = steps == 2 ? 1 : 0;
+    a.ahead[c] = (const float*)((intptr_t)a.in.e[c] + 2 * pe);
+    a.ahead[3 + c] = (const float*)((intptr_t)a.in.h[c] + ph);
+    a.ahead[6 + c] = (const float*)((intptr_t)a.cf.curl[c] + pe);
+    a.behind_e[c] = (float*)((intptr_t)a.out.e[c] - be * pe);
+    a.behind_h[c] = (float*)((intptr_t)a.out.h[c] - bh * ph);
+  }
+}
+
+template <int T>
+void dispatch_march(const mw::MarchArgs& a, int n, int mode, hipStream_t s) {
+  const int blocks = ((a.blocks + 7) / 8) * 8;
+  const dim3 grid(blocks), block(mw::kMarchCols, mw::kMarchRows, 1);
+  if (mode == 2) hipLaunchKernelGGL((mw::march_kernel<T, 2>), grid, block, 0, s, a, n);
+  else if (mode == 1) hipLaunchKernelGGL((mw::march_kernel<T, 1>), grid, block, 0, s, a, n);
+  else hipLaunchKernelGGL((mw::march_kernel<T, 0>), grid, block, 0, s, a, n);
+}
+
+int launch_march(const mw_program* p, const mw_workspace* ws, const mw::MarchArgs& a, int steps, int n, hipStream_t s) {
+  mw::TermSet set{};
+  int64_t cells = 0;
+  for (int f = 0; f < 2; ++f) {
+    const mw_term* t = f ? p->e_terms : p->h_terms;
+    for (int i = 0; i < (f ? p->n_e_terms : p->n_h_terms); ++i) {
+      if (t[i].kind != MW_TERM_SHIFTED) continue;
+      if (set.count == MW_MAX_TERMS) {  // more than one launch's worth (both families full)
+        hipLaunchKernelGGL(mw::march_prepare_kernel, dim3(grid_blocks(cells * steps), set.count), dim3(256), 0, s, set,
+                           mw_aux_line{}, (float*)nullptr, n, steps, p->dt);
+        set.count = 0;
+        cells = 0;
+      }
+      set.t[set.count++] = t[i];
+      cells = std::max<int64_t>(cells, (int64_t)t[i].shape[0] * t[i].shape[1] * t[i].shape[2]);
+    }
+  }
+  const bool line = p->aux.n_e > 0;
+  if (set.count > 0 || line) {
+    hipLaunchKernelGGL(mw::march_prepare_kernel, dim3(std::max(1, grid_blocks(cells * steps)), set.count + (line ? 1 : 0)),
+                       dim3(256), 0, s, set, line ? p->aux : mw_aux_line{}, line ? ws->line_history : nullptr, n, steps,
+                       p->dt);
+    if (int rc = check_launch("march_prepare")) return rc;
+  }
+  const int mode = coef_mode(p->coeffs);
+  if (steps == 2) dispatch_march<2>(a, n, mode, s);
+  else dispatch_march<1>(a, n, mode, s);
+  return check_launch("march");
+}
+#endif  // MW_MARCH
+
 // The single-pass step reads H across a periodic seam from the face on the other
 // side, so a periodic axis must have both faces periodic.
 int check_periodic_pairs(const mw_grid* g) {
@@ -1095,7 +1391,7 @@ int32_t mw_abi_struct_sizes(int64_t* out, int32_t capacity) {
   const int64_t sizes[] = {(int64_t)sizeof(mw_grid),     (int64_t)sizeof(mw_coeffs),   (int64_t)sizeof(mw_cpml),
                            (int64_t)sizeof(mw_fields),   (int64_t)sizeof(mw_pole),     (int64_t)sizeof(mw_ade),
                            (int64_t)sizeof(mw_term),     (int64_t)sizeof(mw_plane_obs), (int64_t)sizeof(mw_program),
-                           (int64_t)sizeof(mw_window),   (int64_t)sizeof(mw_adjoint)};
+                           (int64_t)sizeof(mw_window),   (int64_t)sizeof(mw_adjoint),  (int64_t)sizeof(mw_workspace)};
   const int32_t n = (int32_t)(sizeof(sizes) / sizeof(sizes[0]));
   for (int32_t i = 0; i < n && i < capacity; ++i) out[i] = sizes[i];
   return n;
@@ -1218,6 +1514,10 @@ int mw_update_aux_electric(float* e, const float* h, const float* decay, const f
 }
 
 int mw_run_steps(const mw_program* p, int32_t first, int32_t count, void* stream) {
+  return mw_run_steps_ws(p, nullptr, first, count, stream);
+}
+
+int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, int32_t count, void* stream) {
   if (!p) return fail(MW_ERR_ARGUMENT, "program is NULL");
   int rc;
   const mw_grid* g = &p->grid;
@@ -1238,10 +1538,7 @@ int mw_run_steps(const mw_program* p, int32_t first, int32_t count, void* stream
   const bool staging = p->plane_stage && p->n_planes > 0;
   if (staging && (p->plane_stage_depth < 1 || p->plane_stage_depth > mw::kMaxStageDepth))
     return fail(MW_ERR_ARGUMENT, "plane_stage_depth %d outside [1, %d]", p->plane_stage_depth, mw::kMaxStageDepth);
-  mw::PlaneSet planes{};
-  mw::ZGatherSet zstage{};
-  mw::ZFlushSet zflush{};
-  int64_t plane_cells = 0, zstage_cells = 0, row_floats = 0;
+  StageLayout zonly, every;  // one stage plane per (component, axis, column); planes that repeat one share it
   for (int q = 0; q < p->n_planes; ++q) {
     const mw_plane_obs& o = p->planes[q];
     if (o.component < 0 || o.component > 5 || o.axis < 0 || o.axis > 2 || !o.re || !o.im)
@@ -1249,33 +1546,49 @@ int mw_run_steps(const mw_program* p, int32_t first, int32_t count, void* stream
     int shp[3];
     component_shape(g, o.component, shp);
     if (o.index < 0 || o.index >= shp[o.axis]) return fail(MW_ERR_ARGUMENT, "plane %d index %d outside axis", q, o.index);
-    const int64_t n = o.axis == 0 ? (int64_t)shp[1] * shp[2] : (o.axis == 1 ? (int64_t)shp[0] * shp[2] : (int64_t)shp[0] * shp[1]);
-    if (staging && o.axis == 2) {
-      // one stage plane per (component, column); planes that repeat one share it
-      int z = 0;
-      while (z < zstage.count && !(zstage.comp[z] == o.component && zstage.k[z] == o.index)) ++z;
-      if (z == zstage.count) {
-        zstage.comp[z] = o.component;
-        zstage.k[z] = o.index;
-        zstage.off[z] = row_floats;
-        ++zstage.count;
-        row_floats += n;
-      }
-      zflush.p[zflush.count++] = mw::ZFlushPlane{o.component, 0, zstage.off[z], n, o.re, o.im};
-      zstage_cells = std::max(zstage_cells, n);
+    every.add(g, o);
+    if (staging && o.axis == 2) zonly.add(g, o);
+  }
+  if (zonly.row_floats > 0 && (int64_t)p->plane_stage_depth * zonly.row_floats > p->plane_stage_floats)
+    return fail(MW_ERR_ARGUMENT, "plane_stage holds %lld floats; %d rows of the %d z planes need %lld",
+                (long long)p->plane_stage_floats, p->plane_stage_depth, zonly.count,
+                (long long)((int64_t)p->plane_stage_depth * zonly.row_floats));
+  every.point_off = every.row_floats;
+  every.row_floats += p->n_points;
+#if MW_MARCH
+  const int march = count > 0 ? march_steps(p, ws, every) : 0;
+#else
+  const int march = 0;
+  (void)ws;
+#endif
+  StageLayout& stage = march ? every : zonly;
+  const int64_t row_floats = stage.row_floats;
+  float* const stage_rows = march ? ws->stage : p->plane_stage;
+  const int stage_depth = march ? ws->stage_depth : p->plane_stage_depth;
+  mw::PlaneSet planes{};
+  mw::ZGatherSet zstage{};
+  mw::ZFlushSet zflush{};
+  int64_t plane_cells = 0;
+  for (int q = 0; q < p->n_planes; ++q) {
+    const mw_plane_obs& o = p->planes[q];
+    int shp[3];
+    component_shape(g, o.component, shp);
+    const int64_t n = (int64_t)shp[0] * shp[1] * shp[2] / shp[o.axis];
+    if (march || (staging && o.axis == 2)) {
+      zflush.p[zflush.count++] = mw::ZFlushPlane{o.component, 0, stage.add(g, o), n, o.re, o.im};
     } else {
       planes.p[planes.count++] = o;
       plane_cells = std::max(plane_cells, n);
     }
   }
-  if (zstage.count > 0) {
-    if ((int64_t)p->plane_stage_depth * row_floats > p->plane_stage_floats)
-      return fail(MW_ERR_ARGUMENT, "plane_stage holds %lld floats; %d rows of the %d z planes need %lld",
-                  (long long)p->plane_stage_floats, p->plane_stage_depth, zstage.count,
-                  (long long)((int64_t)p->plane_stage_depth * row_floats));
-    zflush.row_floats = row_floats;
-    zflush.stage = p->plane_stage;
+  zflush.row_floats = row_floats;
+  zflush.stage = stage_rows;
+  for (; zstage.count < zonly.count; ++zstage.count) {
+    zstage.comp[zstage.count] = zonly.planes[zstage.count].component;
+    zstage.k[zstage.count] = zonly.planes[zstage.count].index;
+    zstage.off[zstage.count] = zonly.planes[zstage.count].off;
   }
+  const int64_t zstage_cells = stage.cells;
   if ((p->n_planes > 0 || p->n_points > 0) && (p->nf_obs <= 0 || !p->obs_e_cos || !p->obs_e_sin || !p->obs_h_cos || !p->obs_h_sin))
     return fail(MW_ERR_ARGUMENT, "observer weight tables missing");
   if (p->n_points > 0 && (!p->point_component || !p->point_linear || !p->point_re || !p->point_im))
@@ -1343,6 +1656,70 @@ int mw_run_steps(const mw_program* p, int32_t first, int32_t count, void* stream
     hipLaunchKernelGGL(mw::gather_zplanes_kernel, dim3(j.blocks), dim3(256), 0, s, j.set, j.fs, j.samples);
     return check_launch("gather_zplanes");
   };
+  // fold a block's rows into the sums when it completes or the call ends inside it
+  // (then clear them: rows of steps already folded must add nothing at the block's end)
+  auto fold = [&](int n, bool block_end) {
+    const int row = n % stage_depth;
+    const int64_t off = (int64_t)(n - row) * p->nf_obs;
+    if (zflush.count > 0) {
+      hipLaunchKernelGGL(mw::flush_zstage_kernel, dim3(grid_blocks(zstage_cells), zflush.count), dim3(256), 0, s,
+                         zflush, row + 1, p->nf_obs, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off,
+                         p->obs_h_sin + off);
+      if (int r = check_launch("flush_zstage")) return r;
+    }
+#if MW_MARCH
+    if (march && p->n_points > 0) {
+      hipLaunchKernelGGL(mw::march_points_kernel, dim3(grid_blocks((int64_t)p->n_points * p->nf_obs)), dim3(256), 0, s,
+                         stage_rows + stage.point_off, row_floats, row + 1, p->n_points, p->nf_obs,
+                         p->point_component, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off,
+                         p->obs_h_sin + off, p->point_re, p->point_im);
+      if (int r = check_launch("march_points")) return r;
+    }
+#endif
+    if (block_end) return MW_OK;
+    // the front of the stage, whichever planes its rows held
+    const int64_t folded = (int64_t)(row + 1) * ((march ? ws->stage_floats : p->plane_stage_floats) / stage_depth);
+    hipLaunchKernelGGL(mw::clear_floats_kernel, dim3(grid_blocks(folded)), dim3(256), 0, s, stage_rows, folded);
+    return check_launch("clear_zstage");
+  };
+#if MW_MARCH
+  if (march) {
+    // a state of step n lives in buffer n mod 2, so two-step marches go in pairs
+    // (there and back); a stage block, a multiple of four steps, must not end inside one
+    const bool pairs = march == 2 && count >= 4, aligned = stage.row_floats > 0;
+    mw::MarchArgs one[2], there, back;  // one step from an even / odd one
+    for (int odd = 0; odd < 2; ++odd) build_march_args(p, ws, 1, odd, false, stage, &one[odd]);
+    // the stage rows of the steps a march takes
+    auto staged = [&](mw::MarchArgs& m, int n) -> mw::MarchArgs& {
+      for (int t = 0; t < 2 && aligned; ++t)
+        m.stage[t] = stage_rows + (int64_t)((n + t) % stage_depth) * row_floats;
+      return m;
+    };
+    const int end = first + count;
+    int laid = -1;  // parity that `there` and `back` start from
+    for (int n = first; n < end;) {
+      if (pairs && n + 4 <= end && (!aligned || n % 4 == 0)) {
+        if (laid != (n & 1)) {
+          laid = n & 1;
+          build_march_args(p, ws, 2, laid, false, stage, &there);
+          build_march_args(p, ws, 2, laid, true, stage, &back);
+        }
+        if ((rc = launch_march(p, ws, staged(there, n), 2, n, s)) ||
+            (rc = launch_march(p, ws, staged(back, n + 2), 2, n + 2, s)))
+          return rc;
+        n += 4;
+      } else {
+        if ((rc = launch_march(p, ws, staged(one[n & 1], n), 1, n, s))) return rc;
+        n += 1;
+      }
+      if (aligned) {
+        const bool block_end = n % stage_depth == 0;
+        if ((block_end || n == end) && (rc = fold(n - 1, block_end))) return rc;
+      }
+    }
+    return MW_OK;
+  }
+#endif
   for (int n = first; n < first + count; ++n) {
     if (aux.n_e > 0) {
       hipLaunchKernelGGL(mw::aux_line_h_kernel, dim3((aux.n_e + 254) / 256), dim3(256), 0, s, aux);
@@ -1402,21 +1779,7 @@ int mw_run_steps(const mw_program* p, int32_t first, int32_t count, void* stream
       } else if ((rc = launch_gather(job))) {
         return rc;
       }
-      // fold the block's rows when it completes or the call ends inside it (then
-      // clear them: rows of steps already folded must add nothing at the block's end)
-      if (block_end || call_end) {
-        const int64_t off = (int64_t)(n - row) * p->nf_obs;
-        hipLaunchKernelGGL(mw::flush_zstage_kernel, dim3(grid_blocks(zstage_cells), zflush.count), dim3(256), 0, s,
-                           zflush, row + 1, p->nf_obs, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off,
-                           p->obs_h_sin + off);
-        if ((rc = check_launch("flush_zstage"))) return rc;
-        if (!block_end) {
-          const int64_t folded = (int64_t)(row + 1) * row_floats;
-          hipLaunchKernelGGL(mw::clear_floats_kernel, dim3(grid_blocks(folded)), dim3(256), 0, s, p->plane_stage,
-                             folded);
-          if ((rc = check_launch("clear_zstage"))) return rc;
-        }
-      }
+      if ((block_end || call_end) && (rc = fold(n, block_end))) return rc;
     }
     if (p->n_points > 0) {
       pts = point_set(fs, n);

@@ -245,7 +245,7 @@ class GradientSession:
 
     def __init__(self, plan: FDTDPlan, device="cuda", window=None, stride=None, fused=None, tune=False):
         self.plan = plan
-        self.run = DeviceRun(plan, device, fused=fused)
+        self.run = DeviceRun(plan, device, fused=fused, multi_step=False)  # steps round as their replays do
         if tune and self.run.fused and plan.time_steps >= 200:
             # a few trial steps of each candidate tiling (the run is reset afterwards)
             self.run.autotune(trial_steps=8, xchunks=(0, 6, 8), shell_chunks=(2, 4), z_tilings=(1, 2, 3, 4))

@@ -198,7 +198,7 @@ class BatchGradientSession:
         if len(T) != 1:
             raise ValueError("batched scenes must run the same number of steps")
         self.T = T.pop()
-        self.runs = [DeviceRun(p, device, fused=True) for p in self.plans]
+        self.runs = [DeviceRun(p, device, fused=True, multi_step=False) for p in self.plans]
         self.batch = BatchRun(self.runs, xchunk=xchunk)
         self.batch.graph_steps = int(graph_steps)
         self.windows = list(windows) if windows is not None else [design_window(p) for p in self.plans]

@@ -49,9 +49,12 @@ class DeviceRun:
 
     ``plane_stage_depth`` (0 = off): the samples of z-normal plane monitors are
     copied into a stage of that many steps and added to their sums once per block
-    of steps, instead of the sums being read and written after every step."""
+    of steps, instead of the sums being read and written after every step.
 
-    def __init__(self, plan: FDTDPlan, device="cuda", fused=None, plane_stage_depth=32):
+    ``multi_step=False`` keeps every step a pass of its own, with the rounding of the
+    launches that capture and reverse steps for gradients."""
+
+    def __init__(self, plan: FDTDPlan, device="cuda", fused=None, plane_stage_depth=32, multi_step=True):
         self.plan = plan
         self.device = torch.device(device)
         if self.device.type != "cuda":
@@ -66,6 +69,9 @@ class DeviceRun:
             self._fields.append({c: torch.zeros_like(t) for c, t in self._fields[0].items()})
 
         prog = nat.MwProgram()
+        self._multi = multi = self.fused and bool(multi_step)
+        work = nat.MwWorkspace()  # scratch of passes that take several steps at once
+        work.term_steps = 2 if multi else 1
         g = prog.grid
         g.nx, g.ny, g.nz = nx, ny, nz
         for a in range(3):
@@ -116,6 +122,9 @@ class DeviceRun:
                     alt = torch.zeros_like(t)
                     self._psi_alt[name] = alt
                     prog.psi_h_alt[q - 6] = nat.ptr(alt) if alt.numel() else None
+                elif multi and t.numel():
+                    self.keep.append(torch.empty_like(t))
+                    work.psi_e_alt[q] = nat.ptr(self.keep[-1])
         ad = prog.ade
         ad.dt = plan.dt
         self.ade_state = {}
@@ -171,6 +180,9 @@ class DeviceRun:
             line.decay_h = self._dev(aux["decay_h"])
             line.curl_h = self._dev(aux["curl_h"])
             line.source = self._dev(aux["source"])
+            if multi:
+                self.keep.append(torch.empty(4 * n_e, dtype=torch.float32, device=dev))
+                work.line_history = nat.ptr(self.keep[-1])
 
         # ---- source terms
         cidx = {c: i for i, c in enumerate(COMPONENTS)}
@@ -247,19 +259,28 @@ class DeviceRun:
         prog.n_planes = len(planes)
         # z-normal planes: a row per step of each distinct (component, index)
         self.plane_stage = None
-        z_pairs = {}
-        for q, po in enumerate(planes):
-            if po.axis == 2:
-                z_pairs.setdefault((po.component, po.index), int(self.plane_re[q][0].numel()))
-        z_cells = sum(z_pairs.values())
+        staged = {(po.component, po.axis, po.index): int(self.plane_re[q][0].numel()) for q, po in enumerate(planes)}
+        z_cells = sum(n for (_, axis, _), n in staged.items() if axis == 2)
+        cells = sum(staged.values()) + prog.n_points  # a row of every observer, for passes of several steps
         depth = int(plane_stage_depth)
+        shared = multi and depth > 0 and depth % 4 == 0
         if z_cells > 0 and depth > 0:
             if depth > 64:
                 raise ValueError("plane_stage_depth must be at most 64")
-            self.plane_stage = torch.zeros((depth, z_cells), dtype=torch.float32, device=dev)
+            self.plane_stage = torch.zeros((depth, cells if shared else z_cells), dtype=torch.float32, device=dev)
             prog.plane_stage = nat.ptr(self.plane_stage)
             prog.plane_stage_floats = self.plane_stage.numel()
             prog.plane_stage_depth = depth
+        self._stage = None
+        if multi and cells > 0:
+            if shared and self.plane_stage is not None:
+                self._stage = self.plane_stage
+            else:
+                rows = min(64, max(4, depth // 4 * 4))
+                self._stage = torch.zeros((rows, cells), dtype=torch.float32, device=dev)
+            work.stage = nat.ptr(self._stage)
+            work.stage_floats = self._stage.numel()
+            work.stage_depth = self._stage.shape[0]
 
         # ---- full-field DFT
         self.dft_re, self.dft_im = {}, {}
@@ -276,6 +297,7 @@ class DeviceRun:
                 prog.dft_re[a] = nat.ptr(re)
                 prog.dft_im[a] = nat.ptr(im)
         self.program = prog
+        self.workspace = work if multi else None
         self.step_index = 0
 
     @property
@@ -323,7 +345,8 @@ class DeviceRun:
         term = self._term_common(comp, t)
         term.kind = 1
         term.delay = self._dev(t["delay"], dtype=np.float64)
-        vals = torch.zeros(t["patch"].shape, dtype=torch.float32, device=self.device)
+        # this step's values and, for passes of two steps, the next one's
+        vals = torch.zeros((2 if self._multi else 1,) + t["patch"].shape, dtype=torch.float32, device=self.device)
         self.keep.append(vals)
         term.values = nat.ptr(vals)
         st = t["st"]
@@ -342,7 +365,9 @@ class DeviceRun:
         if count <= 0:
             return self
         with torch.cuda.device(self.device):
-            rc = self.lib.mw_run_steps(ctypes.byref(self.program), self.step_index, count, nat.current_stream())
+            rc = self.lib.mw_run_steps_ws(ctypes.byref(self.program),
+                                          ctypes.byref(self.workspace) if self.workspace is not None else None,
+                                          self.step_index, count, nat.current_stream())
         nat.check(rc, self.lib)
         self.step_index += count
         return self
@@ -442,8 +467,9 @@ class DeviceRun:
                     s["polarization"].zero_()
         for t in self.plane_re + self.plane_im + list(self.dft_re.values()) + list(self.dft_im.values()):
             t.zero_()
-        if self.plane_stage is not None:
-            self.plane_stage.zero_()
+        for t in (self.plane_stage, self._stage):
+            if t is not None:
+                t.zero_()
         if self.aux_e is not None:
             self.aux_e.zero_()
             self.aux_h.zero_()
