@@ -414,11 +414,13 @@ class DeviceRun:
         steps = min(int(trial_steps), max(1, p.time_steps - 1))
         timed = {}
         cands = [(xc, sc, zt) for zt in z_tilings for xc in xchunks for sc in shell_chunks]
+        if self._multi:  # the library's own choice, which may take several steps a pass
+            cands.insert(0, (0, 0, 0))
         cands += [tuple(int(v) for v in c) for c in prefer if tuple(int(v) for v in c) not in cands]
         for cand in cands:
             self.set_tiling(*cand)
             self.reset()
-            self.run(1)  # warm-up
+            self.run(min(4, max(1, p.time_steps - 1)))  # warm-up; passes of several steps start at multiples of 4
             start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             torch.cuda.synchronize()
             start.record()
