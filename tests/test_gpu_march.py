@@ -63,3 +63,24 @@ def test_march_matches_oracle_at_tile_edges(nodes, faces):
         assert torch.equal(t, dev.fields[c]), c
     for a, b in zip(whole.plane_re + [whole.point_re], dev.plane_re + [dev.point_re]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("nf", [1, 2, 3])
+def test_full_field_sums_match_oracle(nf):
+    """Running sums of all E, read in groups of two frequencies: whole and odd groups,
+    on a grid whose tiles and planes end inside."""
+    from oracle.driver import OracleRun
+    from witwin_maxwell_amd.fdtd.runtime import DeviceRun
+    print(f"case: march full-field sums, {nf} frequencies", flush=True)
+    scene, _ = _scene((13, 17, 65), FACES[1], lossy=False)
+    scene.monitors.clear()
+    freqs = tuple(np.linspace(0.9, 1.1, nf) * configs.F0)
+    plan = compile_plan(scene, frequencies=freqs, time_steps=22, window="none", full_field_dft=True)
+    ref, dev = OracleRun(plan).run(), DeviceRun(plan, "cuda").run()
+    torch.cuda.synchronize()
+    assert len(plan.dft_frequencies) == nf
+    for part, sums in enumerate((dev.dft_re, dev.dft_im)):
+        want = {c: np.asarray(ref.dft[c][part]) for c in sums}
+        scale = max(float(np.max(np.abs(v))) for v in want.values())
+        for c, t in sums.items():
+            assert np.max(np.abs(t.double().cpu().numpy() - want[c])) <= 1e-5 * scale, (c, part)

@@ -45,6 +45,7 @@ constexpr int kMarchRows = 16;   // wavefronts (rows) per block
 constexpr int kMarchCols = 64;   // lanes (columns)
 constexpr int kMarchPlanes = 248; // most planes a block walks
 constexpr int kMarchPoints = 64; // point observers a march can take
+constexpr int kMarchDft = 2;    // frequencies whose running sums are read together
 constexpr int kMarchBlocks = 256; // blocks that a march lists one by one
 
 struct MarchBlock {  // one block's tile and planes [x0, x1)
@@ -343,14 +344,14 @@ enum : uint32_t {
   kLayers = 31,
   kFaceYZ = 32,    // its row or some lane on a y or z face
   kWatch = 64,     // an observer of its own samples
-  kFullDft = 128,
   kHeldY = 256, kPecY = 512,  // its row on a held / PEC y face
   kMirror = 1024,             // the grid has a PMC face
 };
 
 // COEF: coefficient mode of the scene (fused.h): 0 general, 1 E curl arrays only,
-// 2 uniform.  `logical` = number of the block.
-template <int T, int COEF>
+// 2 uniform.  DFT: with the full-field running sums (in kernels of their own: beside
+// them the others lost 7-10 % to spilled scalars).  `logical` = number of the block.
+template <int T, int COEF, bool DFT>
 __device__ __forceinline__ void march_block(MarchPtr a, int n, int logical, MarchShared<T>& sh) {
   const int nx = held(a->g.nx), ny = held(a->g.ny), nz = held(a->g.nz);
   const int tiles_z = a->tiles_z, tiles_y = a->tiles_y;
@@ -441,7 +442,6 @@ __device__ __forceinline__ void march_block(MarchPtr a, int n, int logical, Marc
 #pragma unroll
   for (int q = 0; q < 3; ++q)
     if (a->g.bc_lo[q] == MW_BC_PMC || a->g.bc_hi[q] == MW_BC_PMC) met |= kMirror;
-  if (a->nf_dft > 0) met |= kFullDft;
   const uint32_t zh4 = 4u * (uint32_t)max(lzh, 0), ze4 = 4u * (uint32_t)max(lze, 0);
 
   // Source terms.  Where one term of a family meets this wavefront (a plane-wave sheet
@@ -849,6 +849,7 @@ __device__ __forceinline__ void march_block(MarchPtr a, int n, int logical, Marc
   };
   // running DFT of E over plane i: the steps n (`e1`) and, at T = 2, n + 1 (`e2`)
   auto full_dft = [&](int i, const V3& e1, const V3& e2) {
+    if (!jn_ok) return;  // another tile's row; lanes of other tiles read (clamped) and do not write
     const MarchPtr f = fresh(a);
     const int nf = f->nf_dft;
     const uint64_t nxs = (uint64_t)snn * (nx - 1), nys = (uint64_t)smn * nx, nzs = (uint64_t)snm * nx;
@@ -860,29 +861,40 @@ __device__ __forceinline__ void march_block(MarchPtr a, int n, int logical, Marc
       return T == 2 ? __builtin_fmaf(v2, w2, s) : s;
     };
     uint64_t ox = pm(i) * snn + rnn, oy = pn(i) * smn + rmn, oz = pn(i) * snm + rnm;
-    for (int q = 0; q < nf; ++q) {
-      const float c1 = C(w0c)[q], s1 = C(w0s)[q];
-      const float c2 = T == 2 ? C(w0c)[nf + q] : 0.0f, s2 = T == 2 ? C(w0s)[nf + q] : 0.0f;
-      // all six sums of the sample are read before any is written
-      float rx = 0, mx = 0, ry = 0, my = 0, rz = 0, mz = 0;
-      if (dx) { rx = row_load(f->dft_re[0] + ox, kn4); mx = row_load(f->dft_im[0] + ox, kn4); }
-      if (dy) { ry = row_load(f->dft_re[1] + oy, kn4); my = row_load(f->dft_im[1] + oy, kn4); }
-      if (dz) { rz = row_load(f->dft_re[2] + oz, km4); mz = row_load(f->dft_im[2] + oz, km4); }
-      if (dx) {
-        row_store(f->dft_re[0] + ox, kn4, add(rx, e1.x, e2.x, c1, c2));
-        row_store(f->dft_im[0] + ox, kn4, add(mx, e1.x, e2.x, s1, s2));
+    // the sums of a few frequencies are read together before any of them is written:
+    // one wait for memory per group, not per frequency (85^3, three frequencies, 100
+    // steps: 4065 -> 3756 us; groups of four spill registers)
+    for (int q0 = 0; q0 < nf; q0 += kMarchDft) {
+      float r[kMarchDft][3], m[kMarchDft][3];
+#pragma unroll
+      for (int b = 0; b < kMarchDft; ++b) {
+        if (q0 + b >= nf) continue;
+        r[b][0] = row_load(f->dft_re[0] + (ox + b * nxs), kn4); m[b][0] = row_load(f->dft_im[0] + (ox + b * nxs), kn4);
+        r[b][1] = row_load(f->dft_re[1] + (oy + b * nys), kn4); m[b][1] = row_load(f->dft_im[1] + (oy + b * nys), kn4);
+        r[b][2] = row_load(f->dft_re[2] + (oz + b * nzs), km4); m[b][2] = row_load(f->dft_im[2] + (oz + b * nzs), km4);
       }
-      if (dy) {
-        row_store(f->dft_re[1] + oy, kn4, add(ry, e1.y, e2.y, c1, c2));
-        row_store(f->dft_im[1] + oy, kn4, add(my, e1.y, e2.y, s1, s2));
+#pragma unroll
+      for (int b = 0; b < kMarchDft; ++b) {
+        const int q = q0 + b;
+        if (q >= nf) continue;
+        const float c1 = C(w0c)[q], s1 = C(w0s)[q];
+        const float c2 = T == 2 ? C(w0c)[nf + q] : 0.0f, s2 = T == 2 ? C(w0s)[nf + q] : 0.0f;
+        if (dx) {
+          row_store(f->dft_re[0] + (ox + b * nxs), kn4, add(r[b][0], e1.x, e2.x, c1, c2));
+          row_store(f->dft_im[0] + (ox + b * nxs), kn4, add(m[b][0], e1.x, e2.x, s1, s2));
+        }
+        if (dy) {
+          row_store(f->dft_re[1] + (oy + b * nys), kn4, add(r[b][1], e1.y, e2.y, c1, c2));
+          row_store(f->dft_im[1] + (oy + b * nys), kn4, add(m[b][1], e1.y, e2.y, s1, s2));
+        }
+        if (dz) {
+          row_store(f->dft_re[2] + (oz + b * nzs), km4, add(r[b][2], e1.z, e2.z, c1, c2));
+          row_store(f->dft_im[2] + (oz + b * nzs), km4, add(m[b][2], e1.z, e2.z, s1, s2));
+        }
       }
-      if (dz) {
-        row_store(f->dft_re[2] + oz, km4, add(rz, e1.z, e2.z, c1, c2));
-        row_store(f->dft_im[2] + oz, km4, add(mz, e1.z, e2.z, s1, s2));
-      }
-      ox += nxs;
-      oy += nys;
-      oz += nzs;
+      ox += kMarchDft * nxs;
+      oy += kMarchDft * nys;
+      oz += kMarchDft * nzs;
     }
   };
 
@@ -1023,12 +1035,13 @@ __device__ __forceinline__ void march_block(MarchPtr a, int n, int logical, Marc
     }
     // the loads have had the whole plane to arrive; the plane's stores follow
     memory_settled();
+    // the running sums are read ahead of the plane's stores, which retire in order
+    if (DFT && out_e) full_dft(T == 2 ? p - 2 : p, T == 2 ? a2 : e1, T == 2 ? e2 : e1);
     if (T == 1 && out_e) {
       store_h(p < nx1, h1);
       store_e(p < nx1, e1);
       if (flags & (kLayerHy | kLayerHz | kLayerX)) store_psi_h(p, ph);
       if (flags & (kLayerEy | kLayerEz | kLayerX)) store_psi_e(p, pe);
-      if (flags & kFullDft) full_dft(p, e1, e1);
     }
     if (T == 2 && out_e) {
       store_e(p - 2 < nx1, e2);
@@ -1038,10 +1051,7 @@ __device__ __forceinline__ void march_block(MarchPtr a, int n, int logical, Marc
       store_h(p - 1 < nx1, h2);
       if (flags & (kLayerHy | kLayerHz | kLayerX)) store_psi_h(p - 1, q2h);
     }
-    if (T == 2 && out_e) {
-      if (flags & kFullDft) full_dft(p - 2, a2, e2);
-      if (flags & kWatch) observe(1, p - 2, e2, b2);
-    }
+    if (T == 2 && out_e && (flags & kWatch)) observe(1, p - 2, e2, b2);
     if ((flags & kWatch) && s1 && p >= i0 && p < i1) observe(0, p, e1, h1);
     if (T == 2) {
       b3 = b2;
@@ -1084,7 +1094,7 @@ __device__ __forceinline__ void march_block(MarchPtr a, int n, int logical, Marc
 // run of tiles (z fastest, then y), so tiles that share halo rows share an L2.
 __device__ __forceinline__ int march_logical(int w, int blocks) { return (w % 8) * (blocks / 8) + w / 8; }
 
-template <int T, int COEF>
+template <int T, int COEF, bool DFT>
 __global__ __launch_bounds__(kMarchCols* kMarchRows) void march_kernel(MarchArgs args, int n) {
   __shared__ MarchShared<T> sh;
 #ifdef MW_EMULATED_BLOCKS
@@ -1094,7 +1104,7 @@ __global__ __launch_bounds__(kMarchCols* kMarchRows) void march_kernel(MarchArgs
 #endif
   const int logical = march_logical((int)blockIdx.x, (int)gridDim.x);
   if (logical >= a->blocks) return;
-  march_block<T, COEF>(a, n, logical, sh);
+  march_block<T, COEF, DFT>(a, n, logical, sh);
 }
 
 // One thread's share of a step of the TFSF line, H then (after a barrier) E; its

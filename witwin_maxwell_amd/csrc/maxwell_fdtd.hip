@@ -948,13 +948,13 @@ void build_march_args(const mw_program* p, const mw_workspace* ws, int steps, bo
   }
 }
 
-template <int T>
+template <int T, bool DFT>
 void dispatch_march(const mw::MarchArgs& a, int n, int mode, hipStream_t s) {
   const int blocks = ((a.blocks + 7) / 8) * 8;
   const dim3 grid(blocks), block(mw::kMarchCols, mw::kMarchRows, 1);
-  if (mode == 2) hipLaunchKernelGGL((mw::march_kernel<T, 2>), grid, block, 0, s, a, n);
-  else if (mode == 1) hipLaunchKernelGGL((mw::march_kernel<T, 1>), grid, block, 0, s, a, n);
-  else hipLaunchKernelGGL((mw::march_kernel<T, 0>), grid, block, 0, s, a, n);
+  if (mode == 2) hipLaunchKernelGGL((mw::march_kernel<T, 2, DFT>), grid, block, 0, s, a, n);
+  else if (mode == 1) hipLaunchKernelGGL((mw::march_kernel<T, 1, DFT>), grid, block, 0, s, a, n);
+  else hipLaunchKernelGGL((mw::march_kernel<T, 0, DFT>), grid, block, 0, s, a, n);
 }
 
 int launch_march(const mw_program* p, const mw_workspace* ws, const mw::MarchArgs& a, int steps, int n, hipStream_t s) {
@@ -982,8 +982,8 @@ int launch_march(const mw_program* p, const mw_workspace* ws, const mw::MarchArg
     if (int rc = check_launch("march_prepare")) return rc;
   }
   const int mode = coef_mode(p->coeffs);
-  if (steps == 2) dispatch_march<2>(a, n, mode, s);
-  else dispatch_march<1>(a, n, mode, s);
+  if (steps == 2) a.nf_dft > 0 ? dispatch_march<2, true>(a, n, mode, s) : dispatch_march<2, false>(a, n, mode, s);
+  else a.nf_dft > 0 ? dispatch_march<1, true>(a, n, mode, s) : dispatch_march<1, false>(a, n, mode, s);
   return check_launch("march");
 }
 #endif  // MW_MARCH
