@@ -1,11 +1,12 @@
 // CPU emulation of the HIP subset the FDTD library uses, for testing the kernels
 // on the host: device memory is host memory, a launch walks its blocks in order,
-// and each 64-lane wavefront runs on 64 host threads in lockstep wherever the
-// kernels exchange values (__shfl_up/__shfl_down go through a barrier), so the
-// results equal the GPU's up to floating-point contraction.  Built with
-// AddressSanitizer it also checks every index the kernels form.  Graph capture is
+// and a block's threads run in lockstep wherever the kernels exchange values (lane
+// shuffles, ballots, block barriers), so the results equal the GPU's up to
+// floating-point contraction.  Built with AddressSanitizer it also checks every index
+// the kernels form.  Graph capture is
 // reported as unavailable, so batches run their steps one launch at a time.
 #pragma once
+#pragma GCC optimize("no-var-tracking-assignments")  // debug info of the large kernels: 176 -> 66 s of compile time
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
@@ -16,16 +17,22 @@
 #define __host__
 #define __forceinline__ inline
 #define __launch_bounds__(...)
+#define __shared__ static
+#define MW_EMULATED_BLOCKS 1
 #define __builtin_amdgcn_readfirstlane(x) (x)
 struct dim3 { unsigned x, y, z; dim3(unsigned a = 1, unsigned b = 1, unsigned c = 1) : x(a), y(b), z(c) {} };
 struct uint3e { unsigned x, y, z; };
 extern thread_local uint3e blockIdx, threadIdx, blockDim, gridDim;
 inline float atomicAdd(float* p, float v) { float o = *p; *p += v; return o; }
-// lockstep wavefront emulation: each of 64 worker threads is one lane
+// lockstep emulation: lane exchanges and block barriers
 float emu_exchange(float v, int src);
 extern thread_local int emu_lane;
 inline float __shfl_up(float v, unsigned d, int w) { int l = emu_lane; return emu_exchange(v, (l % w) >= (int)d ? l - (int)d : l); }
 inline float __shfl_down(float v, unsigned d, int w) { int l = emu_lane; return emu_exchange(v, (l % w) + (int)d < w ? l + (int)d : l); }
+uint64_t emu_ballot(bool v);
+inline uint64_t __ballot(bool v) { return emu_ballot(v); }
+void emu_barrier();
+inline void __syncthreads() { emu_barrier(); }
 using std::fmax; using std::fmin; using std::exp; using std::cos;
 inline float fminf(float a, float b) { return a < b ? a : b; }
 template <typename T> inline T min(T a, T b) { return a < b ? a : b; }

@@ -2,7 +2,7 @@
 with the float64 oracle.  Run by tests/test_emulated_kernels.py in a child process
 (AddressSanitizer must be preloaded into the interpreter that loads the library).
 
-usage: python run_case.py LIB [CASE ...]   (cases: boxes staged dispersive periodic adjoint; default all)"""
+usage: python run_case.py LIB [CASE ...]   (cases: the names in CASES below; default all)"""
 import contextlib
 import ctypes
 import inspect
@@ -104,6 +104,7 @@ def run(name, scene, kw, steps, tiling, splits=(), stage_depth=32, need_field=Fa
     assert worst <= 1e-5, errs
     if expect:
         assert launches(expect) > before, f"{name}: no {expect} launch"
+    return plan, ref, dev
 
 
 dx = configs.DX
@@ -242,8 +243,74 @@ def case_adjoint():
         assert worst <= 1e-5, errs
 
 
+def march(name, scene, kw, steps, splits=(), **opts):
+    """`run` at the library's own tiling: every step by the tile march, the full-field
+    sums compared as well."""
+    separate = launches("lean_step_kernel") + launches("shell_h_kernel")
+    plan, ref, dev = run(name, scene, kw, steps, (0, 0, 0), splits=splits, expect="march_kernel", **opts)
+    assert launches("lean_step_kernel") + launches("shell_h_kernel") == separate, f"{name}: separate launches"
+    for part, sums in enumerate((dev.dft_re, dev.dft_im)):
+        want = {c: np.asarray(ref.dft[c][part]) for c in sums}
+        for c, err in (family_err({c: t.double().numpy() for c, t in sums.items()}, want) if sums else {}).items():
+            assert err <= 1e-5, (name, "running sums", c, err)
+
+
+def _edge_scene(nodes, faces, lossy):
+    import test_gpu_march as tm
+    scene, freqs = tm._scene(nodes, tm.FACES[faces], lossy)
+    return scene, {"frequencies": freqs, "window": "none"}
+
+
+def case_march():
+    # grids that end inside, at and just past a tile's own rows and columns; every
+    # coefficient mode with PML, mixed, PEC faces; planes of the three axes and a point,
+    # staged eight steps at a time, calls ending inside blocks, in pairs of passes and alone
+    march("march, tile edge, lossy, PML", *_edge_scene((12, 16, 64), 0, True), 15, splits=(1, 12), stage_depth=8)
+    march("march, one past the edge, PML", *_edge_scene((13, 17, 65), 0, False), 9, splits=(3,), stage_depth=4)
+    march("march, one past the edge, mixed", *_edge_scene((13, 17, 65), 1, False), 9, splits=(3,), stage_depth=4)
+    march("march, three tiles each way, lossy, PEC", *_edge_scene((10, 29, 125), 2, True), 6, stage_depth=8)
+    # grids far smaller than a tile, uniform coefficients, PMC faces
+    for nodes in ((2, 2, 2), (3, 2, 5), (2, 7, 3), (5, 3, 67)):
+        s = mw.Scene(domain=mw.Domain(tuple((0.0, (n - 1.01) * dx) for n in nodes)), grid=mw.GridSpec.uniform(dx),
+                     boundary=mw.BoundarySpec.faces(default="pmc"), device="cpu")
+        s.add_source(mw.PointDipole(tuple(0.45 * (n - 1) * dx for n in nodes), (0.5, 0.3, 1.0), profile="ideal",
+                                    source_time=mw.CW(configs.F0)))
+        march("march, small box", s, {"frequencies": (configs.F0,)}, 7, splits=(1,))
+
+
+def case_march_terms():
+    # every kind of source term beside others in the same rows: a soft plane wave (its
+    # time-shifted sheets), dipoles that overlap it and each other, the auxiliary line of
+    # a TFSF box; running sums of all E at three frequencies
+    s, kw = configs.dielectric_boxes(cells=12, pml=5, n_boxes=4, box_range=(3, 6), seed=5)
+    s.domain = mw.Domain(((-6 * dx, 6 * dx), (-7 * dx, 7 * dx), (-24 * dx, 24 * dx)))
+    s.monitors.clear()
+    for z in (0.2 * dx, 1.1 * dx, -22.6 * dx):
+        s.add_source(mw.PointDipole((0.3 * dx, -0.2 * dx, z), (0.4, 0.6, 1.0), profile="ideal",
+                                    source_time=mw.CW(configs.F0)))
+    march("march, plane wave and dipoles", s, dict(kw, frequencies=kw["frequencies"][:3], full_field_dft=True), 10,
+          splits=(3,))
+    t = mw.Scene(domain=mw.Domain(((-6 * dx, 6 * dx), (-10 * dx, 10 * dx), (-9 * dx, 9 * dx))),
+                 grid=mw.GridSpec.uniform(dx), boundary=mw.BoundarySpec.pml(4), device="cpu")
+    t.add_structure(mw.Structure(mw.Box((0, 0, 0), (4 * dx, 5 * dx, 4 * dx)), mw.Material(eps_r=4.0)))
+    t.add_source(mw.PlaneWave((0, -1, 0), (0, 0, 1), source_time=mw.CW(configs.F0),
+                              injection=mw.TFSF(((-3 * dx, 3 * dx), (-7 * dx, 7 * dx), (-6 * dx, 6 * dx)))))
+    t.add_source(mw.PointDipole((4.6 * dx, 8.2 * dx, 7.3 * dx), (0.4, 0.6, 1.0), profile="ideal",
+                                source_time=mw.CW(configs.F0)))
+    t.add_monitor(mw.FluxMonitor("flux", axis="y", position=8 * dx, frequencies=(configs.F0,)))
+    march("march, TFSF box", t, {"frequencies": (configs.F0,), "courant": 0.95, "window": "none"}, 14,
+          splits=(1, 10), stage_depth=8, need_field=True)
+
+
+def case_march_blocks():
+    # a grid large enough for blocks listed one by one, costlier tiles in shorter chunks
+    scene, kw = _edge_scene((262, 17, 125), 0, False)
+    march("march, listed blocks", scene, kw, 5, stage_depth=4)
+
+
 CASES = {"boxes": case_boxes, "staged": case_staged, "dispersive": case_dispersive, "periodic": case_periodic,
-         "adjoint": case_adjoint}
+         "adjoint": case_adjoint, "march": case_march, "march_terms": case_march_terms,
+         "march_blocks": case_march_blocks}
 
 for name in (sys.argv[2:] or list(CASES)):
     CASES[name]()

@@ -14,17 +14,10 @@
 #include "batch.h"
 #include "fused.h"
 #include "shell.h"
+#include "march.h"
 #include "terms.h"
 #include "zedge.h"
 #include "yee.h"
-// The tile march (march.h) exchanges values across a block's wavefronts; a host
-// build without block-wide lockstep leaves it out and takes the separate launches.
-#if defined(__HIP__) || defined(MW_EMULATED_BLOCKS)
-#include "march.h"
-#define MW_MARCH 1
-#else
-#define MW_MARCH 0
-#endif
 
 namespace {
 
@@ -726,7 +719,6 @@ struct StageLayout {
   }
 };
 
-#if MW_MARCH
 // The march's blocks.  A block's plane takes as long as its wavefronts' loads and
 // stores (about 28 cycles of a CU each, whatever they carry: 15 of them a plane for
 // fields and coefficients cost 2.8 us on a full chip at 129^3, 23 with one axis of
@@ -986,7 +978,6 @@ int launch_march(const mw_program* p, const mw_workspace* ws, const mw::MarchArg
   else a.nf_dft > 0 ? dispatch_march<1, true>(a, n, mode, s) : dispatch_march<1, false>(a, n, mode, s);
   return check_launch("march");
 }
-#endif  // MW_MARCH
 
 // The single-pass step reads H across a periodic seam from the face on the other
 // side, so a periodic axis must have both faces periodic.
@@ -1555,12 +1546,7 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
                 (long long)((int64_t)p->plane_stage_depth * zonly.row_floats));
   every.point_off = every.row_floats;
   every.row_floats += p->n_points;
-#if MW_MARCH
   const int march = count > 0 ? march_steps(p, ws, every) : 0;
-#else
-  const int march = 0;
-  (void)ws;
-#endif
   StageLayout& stage = march ? every : zonly;
   const int64_t row_floats = stage.row_floats;
   float* const stage_rows = march ? ws->stage : p->plane_stage;
@@ -1667,7 +1653,6 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
                          p->obs_h_sin + off);
       if (int r = check_launch("flush_zstage")) return r;
     }
-#if MW_MARCH
     if (march && p->n_points > 0) {
       hipLaunchKernelGGL(mw::march_points_kernel, dim3(grid_blocks((int64_t)p->n_points * p->nf_obs)), dim3(256), 0, s,
                          stage_rows + stage.point_off, row_floats, row + 1, p->n_points, p->nf_obs,
@@ -1675,14 +1660,12 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
                          p->obs_h_sin + off, p->point_re, p->point_im);
       if (int r = check_launch("march_points")) return r;
     }
-#endif
     if (block_end) return MW_OK;
     // the front of the stage, whichever planes its rows held
     const int64_t folded = (int64_t)(row + 1) * ((march ? ws->stage_floats : p->plane_stage_floats) / stage_depth);
     hipLaunchKernelGGL(mw::clear_floats_kernel, dim3(grid_blocks(folded)), dim3(256), 0, s, stage_rows, folded);
     return check_launch("clear_zstage");
   };
-#if MW_MARCH
   if (march) {
     // a state of step n lives in buffer n mod 2, so two-step marches go in pairs
     // (there and back); a stage block, a multiple of four steps, must not end inside one
@@ -1719,7 +1702,6 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
     }
     return MW_OK;
   }
-#endif
   for (int n = first; n < first + count; ++n) {
     if (aux.n_e > 0) {
       hipLaunchKernelGGL(mw::aux_line_h_kernel, dim3((aux.n_e + 254) / 256), dim3(256), 0, s, aux);
