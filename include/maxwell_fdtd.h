@@ -299,10 +299,9 @@ typedef struct mw_program {
    * accumulation).  A row holds each distinct (component, index) of the axis-2
    * planes once, in `planes` order, in the sums' layout, so plane_stage needs
    * plane_stage_depth x (sum of their cells) floats.  A call
-   * that ends inside a block folds that block's rows so far and zeroes them, so a
-   * later call that continues the block adds each step once.  The stage must be
-   * zero before the first call and whenever the next call does not start where
-   * the last one ended (a restart or a restored state). */
+   * that ends inside a block folds that block's rows so far, and a later call that
+   * continues the block folds its own, so each step is added once.  A call reads
+   * no row that it has not written: the stage needs no initialisation. */
   float* plane_stage;
   int64_t plane_stage_floats; /* capacity of plane_stage in floats */
   int32_t plane_stage_depth;  /* 1..64 steps per block */
@@ -315,15 +314,15 @@ typedef struct mw_program {
 int mw_run_steps(const mw_program* program, int32_t first, int32_t count, void* stream);
 
 /* Optional buffers of a program that let several steps share one pass over the
- * grid.  Nothing in them outlives a call (`stage` apart, whose rows are zero between
- * calls where it matters): they need no initialisation, and a program's state after a call is where mw_run_steps leaves it.  Two calls that
- * overlap must not share one.  No reference counterpart. */
+ * grid.  Nothing in them outlives a call: they need no initialisation, and a program's
+ * state after a call is where mw_run_steps leaves it.  Two calls that overlap must not
+ * share one.  No reference counterpart. */
 typedef struct mw_workspace {
   float* psi_e_alt[6];  /* same sizes as cpml.psi[0..5] (NULL: no two-step pass with CPML) */
   float* line_history;  /* 4 * aux.n_e floats (NULL: programs with an auxiliary line step singly) */
   int32_t term_steps;   /* steps each SHIFTED term's `values` holds one after another (1 or 2) */
   int32_t stage_depth;  /* rows of `stage`, a multiple of 4 up to 64 */
-  float* stage;         /* zeroed: a row per step of the samples of all observed planes and points, added to
+  float* stage;         /* a row per step of the samples of all observed planes and points, added to
                            the sums a block of rows at a time; may be plane_stage where the depths agree
                            (NULL: programs with observers step singly) */
   int64_t stage_floats;

@@ -308,9 +308,42 @@ def case_march_blocks():
     march("march, listed blocks", scene, kw, 5, stage_depth=4)
 
 
+def case_stage_rows():
+    # steps folded once, whatever the stage's rows hold from before: launches of both
+    # kinds taking turns inside blocks of three steps (the march stages in four), and a
+    # state put back into a run whose rows hold later steps
+    from witwin_maxwell_amd.fdtd.adjoint import restore, snapshot
+    scene, kw = _edge_scene((13, 17, 65), 0, False)
+    scene.device = "cpu"
+    plan = compile_plan(scene, **dict(kw, time_steps=24))
+    ref = OracleRun(plan).run(24)
+    for depth in (3, 4):
+        dev = runtime.DeviceRun(plan, "cpu", plane_stage_depth=depth)
+        for stage in (dev.plane_stage, dev._stage):
+            stage.fill_(float("nan"))
+        for end, z_tiling in ((15, 2), (16, 0), (17, 2), (20, 0), (24, 2)):
+            dev.set_tiling(0, 0, z_tiling).run(end - dev.step_index)
+        errs = _monitor_errs(ref, dev)
+        print(f"stage rows, taking turns, depth {depth}: max err {max(errs.values()):.2e}", flush=True)
+        assert max(errs.values()) <= 1e-5, errs
+    for z_tiling in (0, 2):
+        dev = runtime.DeviceRun(plan, "cpu", plane_stage_depth=8).set_tiling(0, 0, z_tiling)
+        dev.run(14)
+        sums = dev.plane_re + dev.plane_im + [dev.point_re, dev.point_im]
+        state, kept = snapshot(dev), [t.clone() for t in sums]
+        dev.run()
+        want = [t.clone() for t in sums]
+        restore(dev, state, 14)
+        for t, v in zip(sums, kept):
+            t.copy_(v)
+        dev.run()
+        assert all(torch.equal(a, b) for a, b in zip(sums, want)), f"restored state, z_tiling {z_tiling}"
+        print(f"stage rows, restored state, z_tiling {z_tiling}: equal", flush=True)
+
+
 CASES = {"boxes": case_boxes, "staged": case_staged, "dispersive": case_dispersive, "periodic": case_periodic,
          "adjoint": case_adjoint, "march": case_march, "march_terms": case_march_terms,
-         "march_blocks": case_march_blocks}
+         "march_blocks": case_march_blocks, "stage_rows": case_stage_rows}
 
 for name in (sys.argv[2:] or list(CASES)):
     CASES[name]()

@@ -1568,7 +1568,6 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
     }
   }
   zflush.row_floats = row_floats;
-  zflush.stage = stage_rows;
   for (; zstage.count < zonly.count; ++zstage.count) {
     zstage.comp[zstage.count] = zonly.planes[zstage.count].component;
     zstage.k[zstage.count] = zonly.planes[zstage.count].index;
@@ -1642,29 +1641,28 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
     hipLaunchKernelGGL(mw::gather_zplanes_kernel, dim3(j.blocks), dim3(256), 0, s, j.set, j.fs, j.samples);
     return check_launch("gather_zplanes");
   };
-  // fold a block's rows into the sums when it completes or the call ends inside it
-  // (then clear them: rows of steps already folded must add nothing at the block's end)
-  auto fold = [&](int n, bool block_end) {
-    const int row = n % stage_depth;
-    const int64_t off = (int64_t)(n - row) * p->nf_obs;
+  // add the rows of a block's steps up to n into the sums, when the block completes or
+  // the call ends inside it; rows before the call's first step were folded by an earlier
+  // call or hold nothing of this run
+  auto fold = [&](int n) {
+    const int from = std::max(first, n - n % stage_depth), rows = n - from + 1;
+    const float* row = stage_rows + (int64_t)(from % stage_depth) * row_floats;
+    const int64_t off = (int64_t)from * p->nf_obs;
     if (zflush.count > 0) {
+      zflush.stage = row;
       hipLaunchKernelGGL(mw::flush_zstage_kernel, dim3(grid_blocks(zstage_cells), zflush.count), dim3(256), 0, s,
-                         zflush, row + 1, p->nf_obs, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off,
+                         zflush, rows, p->nf_obs, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off,
                          p->obs_h_sin + off);
       if (int r = check_launch("flush_zstage")) return r;
     }
     if (march && p->n_points > 0) {
       hipLaunchKernelGGL(mw::march_points_kernel, dim3(grid_blocks((int64_t)p->n_points * p->nf_obs)), dim3(256), 0, s,
-                         stage_rows + stage.point_off, row_floats, row + 1, p->n_points, p->nf_obs,
-                         p->point_component, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off,
-                         p->obs_h_sin + off, p->point_re, p->point_im);
+                         row + stage.point_off, row_floats, rows, p->n_points, p->nf_obs, p->point_component,
+                         p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off, p->obs_h_sin + off, p->point_re,
+                         p->point_im);
       if (int r = check_launch("march_points")) return r;
     }
-    if (block_end) return MW_OK;
-    // the front of the stage, whichever planes its rows held
-    const int64_t folded = (int64_t)(row + 1) * ((march ? ws->stage_floats : p->plane_stage_floats) / stage_depth);
-    hipLaunchKernelGGL(mw::clear_floats_kernel, dim3(grid_blocks(folded)), dim3(256), 0, s, stage_rows, folded);
-    return check_launch("clear_zstage");
+    return (int)MW_OK;
   };
   if (march) {
     // a state of step n lives in buffer n mod 2, so two-step marches go in pairs
@@ -1695,10 +1693,7 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
         if ((rc = launch_march(p, ws, staged(one[n & 1], n), 1, n, s))) return rc;
         n += 1;
       }
-      if (aligned) {
-        const bool block_end = n % stage_depth == 0;
-        if ((block_end || n == end) && (rc = fold(n - 1, block_end))) return rc;
-      }
+      if (aligned && (n % stage_depth == 0 || n == end) && (rc = fold(n - 1))) return rc;
     }
     return MW_OK;
   }
@@ -1761,7 +1756,7 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
       } else if ((rc = launch_gather(job))) {
         return rc;
       }
-      if ((block_end || call_end) && (rc = fold(n, block_end))) return rc;
+      if ((block_end || call_end) && (rc = fold(n))) return rc;
     }
     if (p->n_points > 0) {
       pts = point_set(fs, n);

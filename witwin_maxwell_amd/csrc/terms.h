@@ -342,12 +342,6 @@ __global__ __launch_bounds__(256) void flush_zstage_kernel(ZFlushSet set, int ro
   }
 }
 
-// p[0, n) = 0 (folded stage rows of a block that a later call continues).
-__global__ __launch_bounds__(256) void clear_floats_kernel(float* __restrict__ p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0f;
-}
-
 // The point observers of one step: the fields that step wrote and the step's
 // weight rows.  Point p adds x * w[f] to its sums (one fused multiply-add each,
 // wherever the sample is taken).

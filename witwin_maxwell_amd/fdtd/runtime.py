@@ -267,7 +267,7 @@ class DeviceRun:
         if z_cells > 0 and depth > 0:
             if depth > 64:
                 raise ValueError("plane_stage_depth must be at most 64")
-            self.plane_stage = torch.zeros((depth, cells if shared else z_cells), dtype=torch.float32, device=dev)
+            self.plane_stage = torch.empty((depth, cells if shared else z_cells), dtype=torch.float32, device=dev)
             prog.plane_stage = nat.ptr(self.plane_stage)
             prog.plane_stage_floats = self.plane_stage.numel()
             prog.plane_stage_depth = depth
@@ -277,7 +277,7 @@ class DeviceRun:
                 self._stage = self.plane_stage
             else:
                 rows = min(64, max(4, depth // 4 * 4))
-                self._stage = torch.zeros((rows, cells), dtype=torch.float32, device=dev)
+                self._stage = torch.empty((rows, cells), dtype=torch.float32, device=dev)
             work.stage = nat.ptr(self._stage)
             work.stage_floats = self._stage.numel()
             work.stage_depth = self._stage.shape[0]
@@ -469,9 +469,6 @@ class DeviceRun:
                     s["polarization"].zero_()
         for t in self.plane_re + self.plane_im + list(self.dft_re.values()) + list(self.dft_im.values()):
             t.zero_()
-        for t in (self.plane_stage, self._stage):
-            if t is not None:
-                t.zero_()
         if self.aux_e is not None:
             self.aux_e.zero_()
             self.aux_h.zero_()
