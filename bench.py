@@ -10,9 +10,9 @@ Prints ONE JSON line.  ``value`` is node-updates per second over exactly
 ``--steps`` timed steps with all inputs resident in HBM; ``protocol`` adds the
 two-point slope (T(2S) - T(S)) / S as the median of several rounds, twice (A/A),
 so the spread of the two medians shows the noise floor; ``roofline`` prices the
-step's algorithmic bytes against 8 TB/s; ``cpu_baseline`` times the float32
-OpenMP transcription of the same update equations (oracle/fdtd_oracle.c) on a
-bounded sample of the same scene on the host cores.
+bytes that a step's launches (or a pass of two steps) must move against 8 TB/s;
+``cpu_baseline`` times the float32 OpenMP transcription of the same update equations
+(oracle/fdtd_oracle.c) on a bounded sample of the same scene on the host cores.
 
 Other workloads: ``--scene vacuum|dispersive`` (forward), ``--workload gradient``
 (one checkpointed design-region gradient), ``--workload batch`` (a design
@@ -144,25 +144,37 @@ def slope_protocol(runner, span, rounds):
             "round_ms_a": [s * 1e3 for s in all_slopes[0]], "round_ms_b": [s * 1e3 for s in all_slopes[1]]}
 
 
+def step_launches(runner):
+    """(kernel label, steps per pass) of what the run takes its steps with: the tile
+    march's passes of two steps, or one step's separate launches."""
+    steps = runner.pass_plan()[0]
+    return (MARCH_KERNEL, steps) if steps > 0 else (STEP_KERNEL, 1)
+
+
 def time_fused(runner, reps):
     """Average duration of one single-pass step (of the passes of two steps, half one's
-    where the runner takes those): the program is copied with
-    its monitors detached, so each step is exactly the step kernels on torch's
+    where the runner takes those).  The separate launches are timed with the program's
+    monitors detached, so each step is exactly the step kernels on torch's
     current stream (with z_tiling 4 the z-end launch runs on a second stream that
-    each step joins back into it), bracketed by HIP events."""
+    each step joins back into it); a march samples its observers in the kernel itself and
+    keeps them.  Bracketed by HIP events."""
     from witwin_maxwell_amd.fdtd import native as nat
     prog = nat.MwProgram()
     ctypes.memmove(ctypes.byref(prog), ctypes.byref(runner.program), ctypes.sizeof(prog))
-    prog.n_planes = 0
-    prog.n_points = 0
+    work = None
+    if runner.pass_plan()[0] > 0:
+        work = ctypes.byref(runner.workspace)
+    else:
+        prog.n_planes = 0
+        prog.n_points = 0
     first = runner.step_index
     reps = min(reps, runner.plan.time_steps - first - 2)
     if reps < 1:
         raise RuntimeError(f"no steps left in the program for the launch timing (at step {first})")
     stream = nat.current_stream()
-    work = ctypes.byref(runner.workspace) if runner.workspace is not None else None
     warm = 4 if reps > 8 else 2
-    reps -= (warm - 2) + (reps - 2) % 4 if reps > 8 else 0  # whole pairs of two-step passes
+    warm += -(first + warm) % 4 if reps > 16 else 0  # pairs of passes begin at multiples of four steps
+    reps -= (warm - 2) + (reps - warm + 2) % 4 if reps > 16 else 0  # whole pairs of passes
     nat.check(runner.lib.mw_run_steps_ws(ctypes.byref(prog), work, first, warm, stream), runner.lib)
     start, end = _events()
     import torch
@@ -574,7 +586,7 @@ def summarize(argv):
 
 
 STEP_KERNEL = "single-pass step (interior, z-end / z-edge, PML-shell H and E, term and aux-line kernels)"
-MARCH_KERNEL = "two-step pass (tile march and term preparation), per step"
+MARCH_KERNEL = "two-step pass (tile march with its observers, and term preparation)"
 _STEP_FAMILIES = ("lean_step_kernel", "shell_h_lean_kernel", "zends_step_kernel", "zedge_step_kernel",
                   "shell_h_kernel", "shell_e_kernel", "shifted_values_kernel", "aux_line_h_kernel",
                   "aux_line_e_kernel")
@@ -732,11 +744,13 @@ def main():
     print(f"[bench] {args.steps} steps in {elapsed:.3f}s ({ms_per_step:.4f} ms/step)", file=sys.stderr, flush=True)
 
     step_bytes, e_bytes, h_bytes = algorithmic_bytes(plan, runner)
+    pass_steps = 1
     if runner.fused:
         # the single-pass step: PML-shell H, lean interior, PML-shell E (+ the tiny
-        # per-step term prep); rocprof splits the time between them
-        dominant, t_dom, b_dom = (MARCH_KERNEL if runner.program.z_tiling == 0 and not runner.plan.dispersive
-                                  else STEP_KERNEL, time_fused(runner, reps), step_bytes)
+        # per-step term prep), rocprof splits the time between them; or a pass of two
+        # steps, which has to move every array once, as a pass of one step does
+        dominant, pass_steps = step_launches(runner)
+        t_dom, b_dom = pass_steps * time_fused(runner, reps), step_bytes
     else:
         t_e = time_kernel(runner, "E", reps)
         t_h = time_kernel(runner, "H", reps)
@@ -749,7 +763,8 @@ def main():
                 "frac": achieved / HBM_PEAK, "traffic": traffic, "kernel": dominant,
                 "kernel_avg_us": t_dom * 1e6, "alg_bytes_per_launch": b_dom,
                 "step_alg_bytes_per_node": step_bytes / nodes,
-                "step_frac": step_bytes * args.steps / elapsed / HBM_PEAK}
+                "steps_per_launch": pass_steps,
+                "step_frac": step_bytes * args.steps / pass_steps / elapsed / HBM_PEAK}
     protocol = None
     if args.slope_steps > 0:
         protocol = slope_protocol(runner, args.slope_steps, args.slope_rounds)

@@ -332,6 +332,13 @@ typedef struct mw_workspace {
 int mw_run_steps_ws(const mw_program* program, const mw_workspace* workspace, int32_t first, int32_t count,
                     void* stream);
 
+/* How mw_run_steps_ws takes the program's steps with that workspace; no device call.
+ * out[0]: steps that share a pass over the grid where a call has four or more in a row
+ * (2; 1 without the buffers for more; 0: launches of the separate kernels), out[1]: the
+ * blocks of such a pass, out[2]: the x planes each of them walks (0: as many as its
+ * tile's cost allows). */
+int mw_pass_plan(const mw_program* program, const mw_workspace* workspace, int32_t* out);
+
 /* ---- adjoint (reverse-mode) ----
  * Design window: the node box [lo, hi) over which dL/d(decay_E) and dL/d(curl_E)
  * are accumulated, each as three z-fastest (hi-lo) boxes, one per E component.

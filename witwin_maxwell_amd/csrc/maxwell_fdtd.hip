@@ -719,6 +719,26 @@ struct StageLayout {
   }
 };
 
+// The stage rows of the program's observers, one stage plane per (component, axis,
+// column); planes that repeat one share it.  `every`: all planes and points (what the
+// march stages), `zonly`: the z planes (what the separate launches stage, if they do).
+int lay_observers(const mw_program* p, bool staging, StageLayout* zonly, StageLayout* every) {
+  if (p->n_planes < 0 || p->n_planes > MW_MAX_PLANES) return fail(MW_ERR_ARGUMENT, "%d planes (max %d)", p->n_planes, MW_MAX_PLANES);
+  for (int q = 0; q < p->n_planes; ++q) {
+    const mw_plane_obs& o = p->planes[q];
+    if (o.component < 0 || o.component > 5 || o.axis < 0 || o.axis > 2 || !o.re || !o.im)
+      return fail(MW_ERR_ARGUMENT, "plane %d descriptor invalid", q);
+    int shp[3];
+    component_shape(&p->grid, o.component, shp);
+    if (o.index < 0 || o.index >= shp[o.axis]) return fail(MW_ERR_ARGUMENT, "plane %d index %d outside axis", q, o.index);
+    every->add(&p->grid, o);
+    if (staging && o.axis == 2) zonly->add(&p->grid, o);
+  }
+  every->point_off = every->row_floats;
+  every->row_floats += p->n_points;
+  return MW_OK;
+}
+
 // The march's blocks.  A block's plane takes as long as its wavefronts' loads and
 // stores (about 28 cycles of a CU each, whatever they carry: 15 of them a plane for
 // fields and coefficients cost 2.8 us on a full chip at 129^3, 23 with one axis of
@@ -732,7 +752,7 @@ struct StageLayout {
 // those: many short blocks even the load out by themselves, and keep the planes in use
 // contiguous (281^3 with CPML: 395 us a step, 478 with one round of equal blocks; 185^3
 // 161, and 146 by weight; with z planes 178 and 185).
-void march_blocks(const mw_program* p, int steps, mw::MarchArgs* out) {
+void march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::MarchArgs* out) {
   mw::MarchArgs& a = *out;
   const mw_grid& g = p->grid;
   const int own_z = mw::kMarchCols - 2 * steps, own_y = mw::kMarchRows - 2 * steps, halo = 2 * steps;
@@ -745,7 +765,7 @@ void march_blocks(const mw_program* p, int steps, mw::MarchArgs* out) {
     if (!c.enabled) return n;
     return std::min({n, c.psi_high_len[e] > 0 ? c.psi_high_start[e] : n, c.psi_high_len[h] > 0 ? c.psi_high_start[h] : n});
   };
-  const int kPlain = 15 + 12 * a.nf_dft, kLayer = 8;
+  const int kPlain = 15 + 12 * p->nf_dft, kLayer = 8;
   const int x_low = std::min(low(0), g.nx), x_high = std::max(high(0, g.nx), x_low), layers = x_low + g.nx - x_high;
   const int tiles = a.tiles_z * a.tiles_y, extra = steps == 2 ? 4 : 1;
   auto even = [&](int chunk) {
@@ -754,14 +774,14 @@ void march_blocks(const mw_program* p, int steps, mw::MarchArgs* out) {
   };
   if (p->xchunk > 0) return even(p->xchunk);
   bool z_planes = false;
-  for (int q = 0; q < a.n_planes; ++q) z_planes = z_planes || a.planes[q].axis == 2;
+  for (int q = 0; q < stage.count; ++q) z_planes = z_planes || stage.planes[q].axis == 2;
   if (c.enabled && (int64_t)tiles * g.nx >= (z_planes ? 512 : 1024) * 16) return even(16);
   // a tile's cost per plane
   auto tile_cost = [&](int z) {
     const int k0 = z * own_z, k1 = std::min(g.nz, k0 + mw::kMarchCols);
     int cost = kPlain + (k0 < low(2) || k1 > high(2, g.nz) ? kLayer : 0);
-    for (int q = 0; q < a.n_planes; ++q)
-      if (a.planes[q].axis == 2 && a.planes[q].index >= k0 && a.planes[q].index < k1) cost += steps;
+    for (int q = 0; q < stage.count; ++q)
+      if (stage.planes[q].axis == 2 && stage.planes[q].index >= k0 && stage.planes[q].index < k1) cost += steps;
     for (int f = 0; f < 2; ++f)
       for (int i = 0; i < (f ? p->n_e_terms : p->n_h_terms); ++i) {
         const mw_term& t = f ? p->e_terms[i] : p->h_terms[i];
@@ -925,7 +945,7 @@ void build_march_args(const mw_program* p, const mw_workspace* ws, int steps, bo
   for (int i = 0; i < stage.count; ++i)
     a.planes[a.n_planes++] = mw::MarchPlane{stage.planes[i].component, stage.planes[i].axis, stage.planes[i].index,
                                             (int)stage.planes[i].off};
-  march_blocks(p, steps, &a);
+  march_blocks(p, stage, steps, &a);
   for (int c = 0; c < 3; ++c) {
     int se[3], sh[3];
     component_shape(&p->grid, c, se);
@@ -1523,29 +1543,17 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
   if ((rc = check_terms(g, p->h_terms, p->n_h_terms, "h_terms", p->total_steps)) ||
       (rc = check_terms(g, p->e_terms, p->n_e_terms, "e_terms", p->total_steps)))
     return rc;
-  if (p->n_planes < 0 || p->n_planes > MW_MAX_PLANES) return fail(MW_ERR_ARGUMENT, "%d planes (max %d)", p->n_planes, MW_MAX_PLANES);
   // planes with axis 2 are staged when the program gives a stage; the others are
   // added to their sums after each step
   const bool staging = p->plane_stage && p->n_planes > 0;
   if (staging && (p->plane_stage_depth < 1 || p->plane_stage_depth > mw::kMaxStageDepth))
     return fail(MW_ERR_ARGUMENT, "plane_stage_depth %d outside [1, %d]", p->plane_stage_depth, mw::kMaxStageDepth);
-  StageLayout zonly, every;  // one stage plane per (component, axis, column); planes that repeat one share it
-  for (int q = 0; q < p->n_planes; ++q) {
-    const mw_plane_obs& o = p->planes[q];
-    if (o.component < 0 || o.component > 5 || o.axis < 0 || o.axis > 2 || !o.re || !o.im)
-      return fail(MW_ERR_ARGUMENT, "plane %d descriptor invalid", q);
-    int shp[3];
-    component_shape(g, o.component, shp);
-    if (o.index < 0 || o.index >= shp[o.axis]) return fail(MW_ERR_ARGUMENT, "plane %d index %d outside axis", q, o.index);
-    every.add(g, o);
-    if (staging && o.axis == 2) zonly.add(g, o);
-  }
+  StageLayout zonly, every;
+  if ((rc = lay_observers(p, staging, &zonly, &every))) return rc;
   if (zonly.row_floats > 0 && (int64_t)p->plane_stage_depth * zonly.row_floats > p->plane_stage_floats)
     return fail(MW_ERR_ARGUMENT, "plane_stage holds %lld floats; %d rows of the %d z planes need %lld",
                 (long long)p->plane_stage_floats, p->plane_stage_depth, zonly.count,
                 (long long)((int64_t)p->plane_stage_depth * zonly.row_floats));
-  every.point_off = every.row_floats;
-  every.row_floats += p->n_points;
   const int march = count > 0 ? march_steps(p, ws, every) : 0;
   StageLayout& stage = march ? every : zonly;
   const int64_t row_floats = stage.row_floats;
@@ -1765,6 +1773,24 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
     }
   }
   if (pts_pending && (rc = launch_points(pts))) return rc;
+  return MW_OK;
+}
+
+int mw_pass_plan(const mw_program* p, const mw_workspace* ws, int32_t* out) {
+  if (!p || !out) return fail(MW_ERR_ARGUMENT, "program or out is NULL");
+  int rc;
+  const mw_grid* g = &p->grid;
+  StageLayout zonly, every;
+  if ((rc = check_grid(g)) || (rc = check_terms(g, p->h_terms, p->n_h_terms, "h_terms", p->total_steps)) ||
+      (rc = check_terms(g, p->e_terms, p->n_e_terms, "e_terms", p->total_steps)) ||
+      (rc = lay_observers(p, false, &zonly, &every)))
+    return rc;
+  mw::MarchArgs a;
+  a.blocks = a.chunk = 0;
+  out[0] = march_steps(p, ws, every);
+  if (out[0] > 0) march_blocks(p, every, out[0], &a);
+  out[1] = a.blocks;
+  out[2] = a.chunk;
   return MW_OK;
 }
 

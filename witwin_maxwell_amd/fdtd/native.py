@@ -117,7 +117,7 @@ STRUCTS = (MwGrid, MwCoeffs, MwCpml, MwFields, MwPole, MwAde, MwTerm, MwPlaneObs
 
 EXPORTS = ("mw_update_magnetic", "mw_update_electric", "mw_add_source_patch", "mw_add_time_shifted_patch",
            "mw_accumulate_dft", "mw_accumulate_plane", "mw_accumulate_points", "mw_run_steps", "mw_run_steps_ws",
-           "mw_capture_steps",
+           "mw_pass_plan", "mw_capture_steps",
            "mw_reverse_steps", "mw_batch_create", "mw_batch_run", "mw_batch_destroy",
            "mw_adjoint_batch_create", "mw_adjoint_batch_capture", "mw_adjoint_batch_reverse",
            "mw_adjoint_batch_destroy", "mw_batch_run_noalloc", "mw_update_pole_current",
@@ -154,6 +154,7 @@ def load_library(path=None):
     lib.mw_accumulate_points.argtypes = [vp, vp, i32, i32, vp, vp, vp, vp, vp]
     lib.mw_run_steps.argtypes = [P(MwProgram), i32, i32, vp]
     lib.mw_run_steps_ws.argtypes = [P(MwProgram), P(MwWorkspace), i32, i32, vp]
+    lib.mw_pass_plan.argtypes = [P(MwProgram), P(MwWorkspace), P(i32)]
     lib.mw_capture_steps.argtypes = [P(MwProgram), i32, i32, P(MwWindow), vp]
     lib.mw_reverse_steps.argtypes = [P(MwProgram), P(MwAdjoint), P(MwWindow), i32, i32, vp]
     lib.mw_batch_create.argtypes = [P(P(MwProgram)), i32, i32, P(vp)]

@@ -372,6 +372,16 @@ class DeviceRun:
         self.step_index += count
         return self
 
+    def pass_plan(self):
+        """(steps that share a pass, blocks of such a pass, planes per block) as the
+        library takes this run's steps; (0, 0, 0): by the separate launches, one step
+        at a time."""
+        out = (ctypes.c_int32 * 3)()
+        nat.check(self.lib.mw_pass_plan(ctypes.byref(self.program),
+                                        ctypes.byref(self.workspace) if self.workspace is not None else None, out),
+                  self.lib)
+        return tuple(out)
+
     def set_tiling(self, xchunk: int = 0, shell_chunk: int = 0, z_tiling: int = 0):
         """Single-pass tiling: x planes per block of the interior and PML-shell
         launches (0 = the library's choice) and how the z ends are tiled (0 or 2:
