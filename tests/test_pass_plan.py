@@ -17,7 +17,7 @@ def lib():
     return native.load_library()
 
 
-def _program(nodes, pml, z_planes=0, lossy=False, dft=0):
+def _program(nodes, pml, z_planes=0, lossy=False, dft=0, plane_wave=False):
     """A single-pass program of that grid with `z_planes` flux planes (six observed
     (component, column) planes each), and a workspace; buffers are never read."""
     fake = ctypes.c_void_p(4096)
@@ -45,6 +45,19 @@ def _program(nodes, pml, z_planes=0, lossy=False, dft=0):
     keep = (native.MwPlaneObs * max(1, len(planes)))(*planes)
     p.planes = ctypes.cast(keep, ctypes.POINTER(native.MwPlaneObs))
     p.n_planes, p.nf_obs, p.nf_dft = len(planes), 8, dft
+    terms = []
+    if plane_wave:  # the two sheets of a soft +z plane wave
+        for c in (0, 4):
+            t = native.MwTerm()
+            t.component, t.kind, t.patch, t.delay, t.values = c, 1, fake, fake, fake
+            for a in range(3):
+                t.offset[a] = pml + 3
+                t.shape[a] = 1 if a == 2 else nodes[a] - 2 * (pml + 3)
+            terms.append(t)
+        held = [(native.MwTerm * 1)(t) for t in terms]
+        p.n_e_terms = p.n_h_terms = 1
+        p.e_terms, p.h_terms = (ctypes.cast(h, ctypes.POINTER(native.MwTerm)) for h in held)
+        keep = (keep, held)
     for q in range(6):
         w.psi_e_alt[q] = fake
     w.line_history, w.term_steps = fake, 2
@@ -89,3 +102,27 @@ def test_benchmark_names_the_launches_a_run_takes(plan, kernel, steps):
         def pass_plan(self):
             return plan
     assert bench.step_launches(Run()) == (getattr(bench, kernel), steps)
+
+
+@pytest.mark.parametrize("nodes,pml,z_planes,lossy,dft,steps,chunk", [
+    # measured on both sides (us a step, two-step passes / separate launches)
+    ((201, 101, 67), 12, 2, False, 0, 0, 0),    # 90 / 71
+    ((401, 65, 125), 8, 2, False, 0, 0, 0),     # 133 / 92
+    ((130, 130, 130), 12, 2, False, 0, 0, 0),   # 88 / 81
+    ((161, 161, 161), 12, 2, False, 0, 2, 0),   # 127 / 149
+    ((281, 105, 105), 12, 2, False, 0, 2, 0),   # 96 / 117
+    ((185, 185, 185), 12, 0, False, 0, 2, 0),   # 174 / 195
+    ((185, 185, 185), 12, 0, True, 0, 0, 0),    # 244 / 209
+    ((201, 101, 67), 12, 0, True, 0, 0, 0),     # 86 / 64
+    ((121, 121, 121), 12, 0, True, 0, 2, 0),    # 66 / 75
+    ((225, 225, 225), 12, 2, False, 0, 2, 0),   # by weight 278, blocks of sixteen planes 324
+    ((249, 249, 249), 12, 2, False, 0, 2, 16),  # 402 and 378
+    ((189, 197, 311), 8, 0, False, 0, 2, 16),   # 272 and 235
+    ((121, 121, 121), 10, 0, False, 1, 2, 0),   # running sums: 58 / 89
+    ((193, 193, 193), 0, 2, True, 0, 2, None),  # no layers: 155 / 201
+])
+def test_route_follows_the_cost_of_both_sides(lib, nodes, pml, z_planes, lossy, dft, steps, chunk):
+    got = _pass_plan(lib, nodes, pml, z_planes, lossy, dft, plane_wave=pml == 12)
+    assert got[0] == steps
+    if chunk is not None:
+        assert got[2] == chunk

@@ -739,6 +739,12 @@ int lay_observers(const mw_program* p, bool staging, StageLayout* zonly, StageLa
   return MW_OK;
 }
 
+// Tiles of `width` samples along an axis of n nodes, the outermost `steps` at each inner
+// side of one computed by its neighbour.
+int march_tiles(int n, int width, int steps) {
+  return std::max(1, (n - 2 * steps + width - 2 * steps - 1) / (width - 2 * steps));
+}
+
 // The march's blocks.  A block's plane takes as long as its wavefronts' loads and
 // stores (about 28 cycles of a CU each, whatever they carry: 15 of them a plane for
 // fields and coefficients cost 2.8 us on a full chip at 129^3, 23 with one axis of
@@ -746,18 +752,26 @@ int lay_observers(const mw_program* p, bool staging, StageLayout* zonly, StageLa
 // z tiles by what lies in them, tile rows at the y ends by their layers, planes at the
 // x ends by theirs.  One block fills a CU, so the grid is cut until every CU has one:
 // the most costly block decides, and costlier tiles get more and shorter chunks.
-// Small grids, where a plane takes its latency whatever lies in it, get equal blocks
-// (73^3 with CPML and two flux planes: 32 us a step, 39 by weight; 105^3 49 and 44).
-// Layered scenes beyond four rounds of blocks of sixteen planes (two with z planes) use
-// those: many short blocks even the load out by themselves, and keep the planes in use
-// contiguous (281^3 with CPML: 395 us a step, 478 with one round of equal blocks; 185^3
-// 161, and 146 by weight; with z planes 178 and 185).
-void march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::MarchArgs* out) {
+// Small grids, where a plane takes its latency whatever lies in it, get equal blocks:
+// passes of two steps below 1536 tile planes (us a step of equal blocks / by weight, CPML,
+// two z flux planes: 73^3, 876 tile planes, 39 / 42; 89^3, 1424, 50 / 52; 105^3, 1890,
+// 58 / 51), passes of one below 600 (CPML 8, a dipole: 61 x 45 x 122, 488, 23.3 / 23.7;
+// 73^3 33.0 / 31.4; 85^3 37 / 32, with one z flux plane 44 / 37; 97^3 42 / 37).
+// Layered scenes beyond 20000 tile planes use blocks of sixteen planes: many short ones
+// even the load out by themselves, and keep the planes in use contiguous (CPML 12, a
+// plane wave, without and with two z flux planes, us a step of sixteen planes / by
+// weight: 241^3, 19280 tile planes, 330 / 273 and 338 / 303; 225 x 225 x 145, 12825, 211 /
+// 174 and 253 / 226; 185 x 265 x 265, 20350, 288 / 274 and 315 / 348; 281 x 185 x 281,
+// 22480, 296 / 340 and 324 / 346; 249^3, 26145, 351 / 389 and 378 / 402), and from 16384
+// on where the weighted blocks come out a tenth costlier (189 x 197 x 311, CPML 8, 235 /
+// 272, its costs 1982 and 2334; 2083 and 2007 for the 241^3 above).
+// Returns the cost of the busiest CU, in those counts.
+int64_t march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::MarchArgs* out) {
   mw::MarchArgs& a = *out;
   const mw_grid& g = p->grid;
-  const int own_z = mw::kMarchCols - 2 * steps, own_y = mw::kMarchRows - 2 * steps, halo = 2 * steps;
-  a.tiles_z = std::max(1, (g.nz - halo + own_z - 1) / own_z);
-  a.tiles_y = std::max(1, (g.ny - halo + own_y - 1) / own_y);
+  const int own_z = mw::kMarchCols - 2 * steps, own_y = mw::kMarchRows - 2 * steps;
+  a.tiles_z = march_tiles(g.nz, mw::kMarchCols, steps);
+  a.tiles_y = march_tiles(g.ny, mw::kMarchRows, steps);
   const mw_cpml& c = p->cpml;
   auto low = [&](int axis) { return c.enabled ? std::max(c.psi_low[axis == 0 ? 2 : axis - 1], c.psi_low[axis == 0 ? 8 : axis + 5]) : 0; };
   auto high = [&](int axis, int n) {
@@ -768,14 +782,6 @@ void march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::
   const int kPlain = 15 + 12 * p->nf_dft, kLayer = 8;
   const int x_low = std::min(low(0), g.nx), x_high = std::max(high(0, g.nx), x_low), layers = x_low + g.nx - x_high;
   const int tiles = a.tiles_z * a.tiles_y, extra = steps == 2 ? 4 : 1;
-  auto even = [&](int chunk) {
-    a.chunk = std::min({chunk, g.nx, mw::kMarchPlanes});
-    a.blocks = tiles * ((g.nx + a.chunk - 1) / a.chunk);
-  };
-  if (p->xchunk > 0) return even(p->xchunk);
-  bool z_planes = false;
-  for (int q = 0; q < stage.count; ++q) z_planes = z_planes || stage.planes[q].axis == 2;
-  if (c.enabled && (int64_t)tiles * g.nx >= (z_planes ? 512 : 1024) * 16) return even(16);
   // a tile's cost per plane
   auto tile_cost = [&](int z) {
     const int k0 = z * own_z, k1 = std::min(g.nz, k0 + mw::kMarchCols);
@@ -792,8 +798,24 @@ void march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::
   auto row_cost = [&](int y) {
     return y * own_y < low(1) || std::min(g.ny, y * own_y + mw::kMarchRows) > high(1, g.ny) ? kLayer : 0;
   };
+  auto even = [&](int chunk) {
+    a.chunk = std::min({chunk, g.nx, mw::kMarchPlanes});
+    const int parts = (g.nx + a.chunk - 1) / a.chunk;
+    a.blocks = tiles * parts;
+    int64_t all = (int64_t)tiles * layers * kLayer, plane = 0;  // a plane of every tile
+    for (int z = 0; z < a.tiles_z; ++z) plane += (int64_t)a.tiles_y * tile_cost(z);
+    for (int y = 0; y < a.tiles_y; ++y) plane += (int64_t)a.tiles_z * row_cost(y);
+    all += plane * (g.nx + (int64_t)extra * parts);
+    return all / mw::kMarchBlocks;
+  };
+  if (p->xchunk > 0) return even(p->xchunk);
+  if (c.enabled && (int64_t)tiles * g.nx >= 20000) return even(16);
   int cost_z[mw::kMarchBlocks], cost_y[mw::kMarchBlocks];
-  bool alike = (int64_t)tiles * g.nx < 1536;
+  struct Kind {  // tiles of one cost: how many, and where the first one's blocks are listed
+    int plane, count, first, blocks;
+  } kinds[mw::kMarchBlocks];
+  int n_kinds = 0;
+  bool alike = (int64_t)tiles * g.nx < (steps == 2 ? 1536 : 600);
   if (tiles <= mw::kMarchBlocks) {
     bool same = layers == 0;
     for (int z = 0; z < a.tiles_z; ++z) cost_z[z] = tile_cost(z);
@@ -802,16 +824,24 @@ void march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::
     for (int y = 1; y < a.tiles_y; ++y) same = same && cost_y[y] == cost_y[0];
     alike = alike || same;
   }
+  auto kind_of = [&](int plane) {
+    for (int q = 0; q < n_kinds; ++q)
+      if (kinds[q].plane == plane) return &kinds[q];
+    kinds[n_kinds] = Kind{plane, 0, 0, 0};
+    return &kinds[n_kinds++];
+  };
+  if (!alike && tiles <= mw::kMarchBlocks)
+    for (int y = 0; y < a.tiles_y; ++y)
+      for (int z = 0; z < a.tiles_z; ++z) kind_of(cost_z[z] + cost_y[y])->count += 1;
   // chunks of a tile for blocks of at most `most`
-  auto chunks = [&](int z, int y, int most) {
-    const int plane = cost_z[z] + cost_y[y], all = g.nx * plane + layers * kLayer, room = most - extra * plane;
+  auto chunks = [&](int plane, int most) {
+    const int all = g.nx * plane + layers * kLayer, room = most - extra * plane;
     return std::min(g.nx, std::max((2 * g.nx + mw::kMarchPlanes - 1) / mw::kMarchPlanes,
                                    room > 0 ? (all + room - 1) / room : g.nx));
   };
   auto total = [&](int most) {
     int n = 0;
-    for (int z = 0; z < a.tiles_z; ++z)
-      for (int y = 0; y < a.tiles_y; ++y) n += chunks(z, y, most);
+    for (int q = 0; q < n_kinds; ++q) n += kinds[q].count * chunks(kinds[q].plane, most);
     return n;
   };
   int lo = 0, hi = (g.nx + extra) * (kPlain + 64) + layers * kLayer + 64 * MW_MAX_TERMS;
@@ -833,31 +863,71 @@ void march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::
     const int mid = (lo + hi) / 2;
     (total(mid) <= mw::kMarchBlocks ? hi : lo) = mid;
   }
+  if (c.enabled && (int64_t)tiles * g.nx >= 16384 && 10 * hi > 11 * even(16)) return even(16);
   a.chunk = 0;
   a.blocks = 0;
   for (int y = 0; y < a.tiles_y; ++y)
     for (int z = 0; z < a.tiles_z; ++z) {
-      const int n = chunks(z, y, hi), plane = cost_z[z] + cost_y[y], all = g.nx * plane + layers * kLayer;
+      Kind& k = *kind_of(cost_z[z] + cost_y[y]);
+      const int n = chunks(k.plane, hi), all = g.nx * k.plane + layers * kLayer;
+      if (k.blocks > 0) {  // as the first tile of its cost
+        for (int q = 0; q < k.blocks; ++q) {
+          const mw::MarchBlock& f = a.list[k.first + q];
+          a.list[a.blocks++] = mw::MarchBlock{f.x0, f.x1, (uint8_t)y, (uint8_t)z};
+        }
+        continue;
+      }
+      k.first = a.blocks;
       int x = 0;
       int64_t spent = 0;
       for (int q = 0; q < n && x < g.nx; ++q) {
         const int x0 = x;
         for (; x < g.nx && (x == x0 || spent * n < (int64_t)all * (q + 1)); ++x)
-          spent += plane + (x < x_low || x >= x_high ? kLayer : 0);
+          spent += k.plane + (x < x_low || x >= x_high ? kLayer : 0);
         if (q == n - 1) x = g.nx;
         a.list[a.blocks++] = mw::MarchBlock{(uint16_t)x0, (uint16_t)x, (uint8_t)y, (uint8_t)z};
       }
+      k.blocks = a.blocks - k.first;
     }
   std::sort(a.list, a.list + a.blocks, [](const mw::MarchBlock& l, const mw::MarchBlock& r) {
     const int dl = l.x0 + l.x1, dr = r.x0 + r.x1;
     return dl != dr ? dl < dr : l.y != r.y ? l.y < r.y : l.z < r.z;
   });
+  return hi;
+}
+
+// Do two-step passes, their busiest CU at `cost`, beat the separate launches of a
+// layered scene?  Both sides were measured on 118 scenes of CPML 8-12 from 105^3 to 281^3
+// nodes (cubes, slabs of 67-89 columns, rods), with a dipole or a plane wave, with and
+// without flux planes, lossless and lossy.  A march takes 0.115 us a step and unit of
+// cost (0.10-0.14), 1.5 times that where conductivity makes the coefficients general; the
+// separate launches 28 us a step, 23 us per million nodes (17-30) and 50 us per million samples
+// of z planes.  The side this picks is on average 0.5 % slower than the faster one, at
+// most 13 %.  us a step, march / separate: 201 x 101 x 67 with two z flux planes 90 / 71,
+// 161^3 127 / 149, 185^3 209 / 211, 225^3 278 / 324; 401 x 65 x 125 without planes 99 / 84;
+// lossy 201 x 101 x 67 86 / 64, 201^3 270 / 259, 121^3 66 / 75, 74^3 46 / 43.  Smaller
+// grids are left to the march (73^3 38 / 43), and so are scenes without layers (129^3 PEC
+// 32 / 47, lossy 47 / 55) and with running sums (121^3, one frequency, 58 / 89).
+// `two` takes the blocks of a two-step pass where the answer needs them.
+bool march_pays(const mw_program* p, const StageLayout& stage, mw::MarchArgs* two) {
+  const int64_t tile_planes = (int64_t)march_tiles(p->grid.nz, mw::kMarchCols, 2) *
+                              march_tiles(p->grid.ny, mw::kMarchRows, 2) * p->grid.nx;
+  const bool general = coef_mode(p->coeffs) == 0;
+  if (!p->cpml.enabled || p->nf_dft > 0 || tile_planes < (general ? 700 : 2048)) return true;
+  const int64_t cost = march_blocks(p, stage, 2, two);
+  int64_t samples = 0;
+  for (int q = 0; q < stage.count; ++q)
+    if (stage.planes[q].axis == 2) samples += stage.planes[q].cells;
+  const double nodes = (double)p->grid.nx * p->grid.ny * p->grid.nz;
+  const double march_ns = 115.0 * cost * (general ? 1.5 : 1.0);
+  return march_ns < 28e3 + 0.023 * nodes + 0.050 * samples;
 }
 
 // May the program's steps be taken by the march, one at a time (1) or two (2), or
 // not at all (0)?  Explicit z tilings ask for the separate launches; periodic faces
 // need H from across the seam, which only their shell pass reads.
-int march_steps(const mw_program* p, const mw_workspace* ws, const StageLayout& stage) {
+int march_steps(const mw_program* p, const mw_workspace* ws, const StageLayout& stage, mw::MarchArgs* two) {
+  two->blocks = 0;
   if (!ws || !p->fused || p->z_tiling != 0 || p->n_points > mw::kMarchPoints) return 0;
   if (grid_periodic(p->grid)) return 0;
   if (p->has_ade && p->ade.count[0] + p->ade.count[1] + p->ade.count[2] > 0) return 0;
@@ -866,15 +936,6 @@ int march_steps(const mw_program* p, const mw_workspace* ws, const StageLayout& 
       (!ws->stage || ws->stage_depth < 4 || ws->stage_depth % 4 != 0 || ws->stage_depth > mw::kMaxStageDepth ||
        stage.row_floats >= (1 << 30) || ws->stage_depth * stage.row_floats > ws->stage_floats))
     return 0;
-  // z planes in a CPML scene of medium size: every block of a z tile waits for the
-  // wavefronts that store samples, and the blocks are too few to even it out (137^3 with
-  // two flux planes: 83 us a step, 75 by the separate launches; 105^3 44 against 48,
-  // 185^3 178 against 179)
-  if (p->cpml.enabled) {
-    const int64_t tiles = (int64_t)((p->grid.nz + 55) / 60) * ((p->grid.ny + 7) / 12) * p->grid.nx;
-    for (int q = 0; q < stage.count && tiles >= 4096 && tiles < 8192; ++q)
-      if (stage.planes[q].axis == 2) return 0;
-  }
   // byte offsets within a component (two planes past its end included) are 32-bit
   if (((int64_t)p->grid.nx + 3) * p->grid.ny * p->grid.nz * 4 >= (int64_t(1) << 32)) return 0;
   if (p->cpml.enabled) {  // the march keeps one slab layout per family and axis
@@ -898,6 +959,7 @@ int march_steps(const mw_program* p, const mw_workspace* ws, const StageLayout& 
     }
   }
   if (p->aux.n_e > 0 && !ws->line_history) return 0;
+  if (!march_pays(p, stage, two)) return 0;
   if (shifted && ws->term_steps < 2) return 1;
   if (p->cpml.enabled)
     for (int q = 0; q < 6; ++q)
@@ -907,9 +969,10 @@ int march_steps(const mw_program* p, const mw_workspace* ws, const StageLayout& 
 
 // Arguments of a march of `steps` steps that start at an even (odd = false) or odd
 // step, reading the state where that step's state lives; `back`: reading the other
-// buffers instead and writing these (the second of two two-step marches).
+// buffers instead and writing these (the second of two two-step marches).  `blocks`:
+// arguments that hold the blocks of such a march.
 void build_march_args(const mw_program* p, const mw_workspace* ws, int steps, bool odd, bool back,
-                      const StageLayout& stage, mw::MarchArgs* out) {
+                      const StageLayout& stage, const mw::MarchArgs& blocks, mw::MarchArgs* out) {
   mw::MarchArgs& a = *out;
   memset(&a, 0, sizeof(a));
   a.g = p->grid;
@@ -945,7 +1008,11 @@ void build_march_args(const mw_program* p, const mw_workspace* ws, int steps, bo
   for (int i = 0; i < stage.count; ++i)
     a.planes[a.n_planes++] = mw::MarchPlane{stage.planes[i].component, stage.planes[i].axis, stage.planes[i].index,
                                             (int)stage.planes[i].off};
-  march_blocks(p, stage, steps, &a);
+  a.tiles_z = blocks.tiles_z;
+  a.tiles_y = blocks.tiles_y;
+  a.blocks = blocks.blocks;
+  a.chunk = blocks.chunk;
+  if (a.chunk == 0) memcpy(a.list, blocks.list, sizeof(a.list));
   for (int c = 0; c < 3; ++c) {
     int se[3], sh[3];
     component_shape(&p->grid, c, se);
@@ -1554,7 +1621,9 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
     return fail(MW_ERR_ARGUMENT, "plane_stage holds %lld floats; %d rows of the %d z planes need %lld",
                 (long long)p->plane_stage_floats, p->plane_stage_depth, zonly.count,
                 (long long)((int64_t)p->plane_stage_depth * zonly.row_floats));
-  const int march = count > 0 ? march_steps(p, ws, every) : 0;
+  mw::MarchArgs blocks[3];  // the blocks of passes of one and two steps, once they are known
+  blocks[1].blocks = 0;
+  const int march = count > 0 ? march_steps(p, ws, every, &blocks[2]) : 0;
   StageLayout& stage = march ? every : zonly;
   const int64_t row_floats = stage.row_floats;
   float* const stage_rows = march ? ws->stage : p->plane_stage;
@@ -1677,7 +1746,11 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
     // (there and back); a stage block, a multiple of four steps, must not end inside one
     const bool pairs = march == 2 && count >= 4, aligned = stage.row_floats > 0;
     mw::MarchArgs one[2], there, back;  // one step from an even / odd one
-    for (int odd = 0; odd < 2; ++odd) build_march_args(p, ws, 1, odd, false, stage, &one[odd]);
+    bool built[2] = {false, false};
+    auto build = [&](int steps, bool odd, bool there_and_back, mw::MarchArgs* out) {
+      if (blocks[steps].blocks == 0) march_blocks(p, stage, steps, &blocks[steps]);
+      build_march_args(p, ws, steps, odd, there_and_back, stage, blocks[steps], out);
+    };
     // the stage rows of the steps a march takes
     auto staged = [&](mw::MarchArgs& m, int n) -> mw::MarchArgs& {
       for (int t = 0; t < 2 && aligned; ++t)
@@ -1690,14 +1763,16 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
       if (pairs && n + 4 <= end && (!aligned || n % 4 == 0)) {
         if (laid != (n & 1)) {
           laid = n & 1;
-          build_march_args(p, ws, 2, laid, false, stage, &there);
-          build_march_args(p, ws, 2, laid, true, stage, &back);
+          build(2, laid, false, &there);
+          build(2, laid, true, &back);
         }
         if ((rc = launch_march(p, ws, staged(there, n), 2, n, s)) ||
             (rc = launch_march(p, ws, staged(back, n + 2), 2, n + 2, s)))
           return rc;
         n += 4;
       } else {
+        if (!built[n & 1]) build(1, n & 1, false, &one[n & 1]);
+        built[n & 1] = true;
         if ((rc = launch_march(p, ws, staged(one[n & 1], n), 1, n, s))) return rc;
         n += 1;
       }
@@ -1786,8 +1861,8 @@ int mw_pass_plan(const mw_program* p, const mw_workspace* ws, int32_t* out) {
       (rc = lay_observers(p, false, &zonly, &every)))
     return rc;
   mw::MarchArgs a;
+  out[0] = march_steps(p, ws, every, &a);
   a.blocks = a.chunk = 0;
-  out[0] = march_steps(p, ws, every);
   if (out[0] > 0) march_blocks(p, every, out[0], &a);
   out[1] = a.blocks;
   out[2] = a.chunk;
