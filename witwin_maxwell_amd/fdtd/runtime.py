@@ -384,9 +384,10 @@ class DeviceRun:
 
     def set_tiling(self, xchunk: int = 0, shell_chunk: int = 0, z_tiling: int = 0):
         """Single-pass tiling: x planes per block of the interior and PML-shell
-        launches (0 = the library's choice) and how the z ends are tiled (0 or 2:
-        interior tiles aligned to the z PML slabs, z ends in the per-cell shell;
-        1: z-edge tiles beside the interior tiles; 3: aligned interior tiles and
+        launches (0 = the library's choice) and how the z ends are tiled (0: the
+        library's own way, where it pays passes of several steps, in blocks of
+        ``xchunk`` planes if given, else as 2; 2: interior tiles aligned to the z PML
+        slabs, z ends in the per-cell shell; 1: z-edge tiles beside the interior tiles; 3: aligned interior tiles and
         both z ends of two rows per wavefront, where they fit, else as 2; 4: as 3
         with the z-end launch on a second stream beside the interior launch)."""
         self.program.xchunk = int(xchunk)
@@ -401,7 +402,9 @@ class DeviceRun:
         within ``margin`` of the fastest, the first of ``prefer`` (tilings the
         caller has other data for) is taken.  The choice is cached per (shape,
         CPML, dispersive, DFT) signature for the rest of the process and in the
-        JSON file named by WITWIN_MAXWELL_AMD_TUNE_CACHE, when set.  Returns
+        JSON file named by WITWIN_MAXWELL_AMD_TUNE_CACHE, when set; runs whose
+        steps share passes at the library's own tiling (0, 0, 0) keep theirs apart,
+        by those passes and the observers they sample.  Returns
         (xchunk, shell_chunk, z_tiling)."""
         import json
         import os
@@ -409,6 +412,13 @@ class DeviceRun:
             return (0, 0, 0)
         p = self.plan
         sig = f"single|{p.shape}|{int(p.uses_cpml)}|{int(p.dispersive)}|{len(p.dft_frequencies)}"
+        cands = [(xc, sc, zt) for zt in z_tilings for xc in xchunks for sc in shell_chunks]
+        passes = self.set_tiling(0, 0, 0).pass_plan()
+        if passes[0] > 0:  # the library's own choice takes several steps a pass
+            axes = [self._planes[q].axis for q in range(self.program.n_planes)]
+            sig += f"|passes {passes}|{[axes.count(a) for a in range(3)]}|{self.program.n_points}"
+            cands.insert(0, (0, 0, 0))
+        cands += [tuple(int(v) for v in c) for c in prefer if tuple(int(v) for v in c) not in cands]
         path = os.environ.get("WITWIN_MAXWELL_AMD_TUNE_CACHE")
         table = {}
         if cache and path and os.path.exists(path):
@@ -417,29 +427,27 @@ class DeviceRun:
         if cache and sig in _TUNED:
             self.set_tiling(*_TUNED[sig])
             return tuple(_TUNED[sig])
-        if sig in table:
+        # an untimed (0, 0, 0) is what a run with passes of several steps once left there
+        if sig in table and (tuple(table[sig]) in cands or any(table[sig])):
             _TUNED[sig] = tuple(table[sig])
             self.set_tiling(*table[sig])
             return tuple(table[sig])
-        steps = min(int(trial_steps), max(1, p.time_steps - 1))
+        warm = min(4, max(1, p.time_steps - 1))  # passes of several steps start at multiples of 4
+        steps = min(int(trial_steps), p.time_steps - warm)
         timed = {}
-        cands = [(xc, sc, zt) for zt in z_tilings for xc in xchunks for sc in shell_chunks]
-        if self._multi:  # the library's own choice, which may take several steps a pass
-            cands.insert(0, (0, 0, 0))
-        cands += [tuple(int(v) for v in c) for c in prefer if tuple(int(v) for v in c) not in cands]
         for cand in cands:
             self.set_tiling(*cand)
             self.reset()
-            self.run(min(4, max(1, p.time_steps - 1)))  # warm-up; passes of several steps start at multiples of 4
+            self.run(warm)
             start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             torch.cuda.synchronize()
             start.record()
-            self.run(min(steps, p.time_steps - self.step_index))
+            self.run(steps)
             end.record()
             end.synchronize()
             timed[cand] = start.elapsed_time(end)
         # ms per step of every candidate, for the caller's records
-        self.autotune_timings = {c: t / steps for c, t in timed.items()}
+        self.autotune_timings = {c: t / max(1, steps) for c, t in timed.items()}
         best = min(timed, key=timed.get)
         for c in prefer:
             c = tuple(int(v) for v in c)
