@@ -341,9 +341,50 @@ def case_stage_rows():
         print(f"stage rows, restored state, z_tiling {z_tiling}: equal", flush=True)
 
 
+def case_scratch():
+    # scratch of shared passes: only where the library takes a run's steps that way, given
+    # back by a batch's scenes, made again when one of them runs alone
+    from witwin_maxwell_amd.fdtd.batch import BatchRun
+    scene, kw = _edge_scene((13, 17, 65), 0, False)
+    scene.device = "cpu"
+    plan = compile_plan(scene, **dict(kw, time_steps=9))
+    z_cells = sum(t[0].numel() for (_, a, _), t in zip(plan.observers.planes, runtime.DeviceRun(plan, "cpu").plane_re)
+                  if a == "z")
+    run_, single = runtime.DeviceRun(plan, "cpu"), runtime.DeviceRun(plan, "cpu", multi_step=False)
+    assert run_.pass_plan()[0] == 2 and run_._scratch and run_.plane_stage is run_._stage
+    assert single.workspace is None and not single._scratch and single.plane_stage.shape[1] == z_cells
+    refused = {"periodic": mw.BoundarySpec.faces(default="pml", x="periodic", num_layers=4), "poles": scene.boundary}
+    for name, boundary in refused.items():
+        other, _ = _edge_scene((13, 17, 65), 0, False)
+        other.device, other.boundary = "cpu", boundary
+        if name == "poles":
+            other.add_structure(mw.Structure(mw.Box((0, 0, 0), (4 * dx, 4 * dx, 4 * dx)),
+                                             mw.Material(eps_r=2.0, drude_poles=(mw.DrudePole(1e14, 1e13),))))
+        dev = runtime.DeviceRun(compile_plan(other, **dict(kw, time_steps=9)), "cpu")
+        assert dev.workspace is None and not dev._scratch and dev._stage is None, name
+        assert dev.plane_stage.shape[1] == sum(t[0].numel() for (_, a, _), t in
+                                               zip(dev.plan.observers.planes, dev.plane_re) if a == "z")
+    want = run_.run()
+    members = [runtime.DeviceRun(plan, "cpu") for _ in range(2)]
+    members[0].run(4)
+    members[0].reset()
+    batch = BatchRun(members)
+    assert all(m.workspace is None and not m._scratch and m._stage is None for m in members)
+    batch.run(2)
+    batch.reset()
+    members[1].run()
+    assert members[1].pass_plan()[0] == 2
+    for c in COMPONENTS:
+        assert torch.equal(members[1].fields[c], want.fields[c]), c
+    for a, b in zip(members[1].plane_re + [members[1].point_re], want.plane_re + [want.point_re]):
+        assert torch.equal(a, b)
+    print("scratch: as the library takes the steps", flush=True)
+
+
 CASES = {"boxes": case_boxes, "staged": case_staged, "dispersive": case_dispersive, "periodic": case_periodic,
          "adjoint": case_adjoint, "march": case_march, "march_terms": case_march_terms,
-         "march_blocks": case_march_blocks, "stage_rows": case_stage_rows}
+         "march_blocks": case_march_blocks, "stage_rows": case_stage_rows,
+         "scratch": case_scratch}
 
 for name in (sys.argv[2:] or list(CASES)):
     CASES[name]()

@@ -13,7 +13,7 @@ import pytest
 
 from test_emulated_kernels import CSRC, EMU, ROOT, _asan_runtime
 
-GROUPS = ("march", "march_terms", "march_blocks", "stage_rows")
+GROUPS = ("march", "march_terms", "march_blocks", "stage_rows", "scratch")
 
 
 @pytest.fixture(scope="module")

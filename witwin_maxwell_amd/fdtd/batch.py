@@ -41,6 +41,8 @@ class BatchRun:
         for r in self.runs:
             if not r.fused:
                 raise ValueError("batched scenes must use the single-pass step")
+        for r in self.runs:
+            r.drop_workspace()
         self.lib = self.runs[0].lib
         self.xchunk = int(xchunk)
         self._handle = None

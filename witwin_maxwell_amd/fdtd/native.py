@@ -107,6 +107,9 @@ class MwAdjoint(ctypes.Structure):
                 ("g_dft_re", vp * 3), ("g_dft_im", vp * 3)]
 
 
+BC_PERIODIC = 2  # MW_BC_PERIODIC
+
+
 class MwWorkspace(ctypes.Structure):
     _fields_ = [("psi_e_alt", vp * 6), ("line_history", vp), ("term_steps", ctypes.c_int32),
                 ("stage_depth", ctypes.c_int32), ("stage", vp), ("stage_floats", ctypes.c_int64)]

@@ -69,9 +69,9 @@ class DeviceRun:
             self._fields.append({c: torch.zeros_like(t) for c, t in self._fields[0].items()})
 
         prog = nat.MwProgram()
-        self._multi = multi = self.fused and bool(multi_step)
-        work = nat.MwWorkspace()  # scratch of passes that take several steps at once
-        work.term_steps = 2 if multi else 1
+        # may steps share a pass at all; the library decides over the rest (`_add_workspace`)
+        self._multi = (self.fused and bool(multi_step) and nat.BC_PERIODIC not in (*plan.bc_lo, *plan.bc_hi)
+                       and not any(plan.ade[c]["poles"] for c in ("Ex", "Ey", "Ez")))
         g = prog.grid
         g.nx, g.ny, g.nz = nx, ny, nz
         for a in range(3):
@@ -122,9 +122,6 @@ class DeviceRun:
                     alt = torch.zeros_like(t)
                     self._psi_alt[name] = alt
                     prog.psi_h_alt[q - 6] = nat.ptr(alt) if alt.numel() else None
-                elif multi and t.numel():
-                    self.keep.append(torch.empty_like(t))
-                    work.psi_e_alt[q] = nat.ptr(self.keep[-1])
         ad = prog.ade
         ad.dt = plan.dt
         self.ade_state = {}
@@ -180,9 +177,6 @@ class DeviceRun:
             line.decay_h = self._dev(aux["decay_h"])
             line.curl_h = self._dev(aux["curl_h"])
             line.source = self._dev(aux["source"])
-            if multi:
-                self.keep.append(torch.empty(4 * n_e, dtype=torch.float32, device=dev))
-                work.line_history = nat.ptr(self.keep[-1])
 
         # ---- source terms
         cidx = {c: i for i, c in enumerate(COMPONENTS)}
@@ -257,31 +251,6 @@ class DeviceRun:
         self._planes = (nat.MwPlaneObs * max(1, len(planes)))(*planes)
         prog.planes = ctypes.cast(self._planes, ctypes.POINTER(nat.MwPlaneObs))
         prog.n_planes = len(planes)
-        # z-normal planes: a row per step of each distinct (component, index)
-        self.plane_stage = None
-        staged = {(po.component, po.axis, po.index): int(self.plane_re[q][0].numel()) for q, po in enumerate(planes)}
-        z_cells = sum(n for (_, axis, _), n in staged.items() if axis == 2)
-        cells = sum(staged.values()) + prog.n_points  # a row of every observer, for passes of several steps
-        depth = int(plane_stage_depth)
-        shared = multi and depth > 0 and depth % 4 == 0
-        if z_cells > 0 and depth > 0:
-            if depth > 64:
-                raise ValueError("plane_stage_depth must be at most 64")
-            self.plane_stage = torch.empty((depth, cells if shared else z_cells), dtype=torch.float32, device=dev)
-            prog.plane_stage = nat.ptr(self.plane_stage)
-            prog.plane_stage_floats = self.plane_stage.numel()
-            prog.plane_stage_depth = depth
-        self._stage = None
-        if multi and cells > 0:
-            if shared and self.plane_stage is not None:
-                self._stage = self.plane_stage
-            else:
-                rows = min(64, max(4, depth // 4 * 4))
-                self._stage = torch.empty((rows, cells), dtype=torch.float32, device=dev)
-            work.stage = nat.ptr(self._stage)
-            work.stage_floats = self._stage.numel()
-            work.stage_depth = self._stage.shape[0]
-
         # ---- full-field DFT
         self.dft_re, self.dft_im = {}, {}
         if plan.dft_frequencies:
@@ -297,8 +266,66 @@ class DeviceRun:
                 prog.dft_re[a] = nat.ptr(re)
                 prog.dft_im[a] = nat.ptr(im)
         self.program = prog
-        self.workspace = work if multi else None
         self.step_index = 0
+
+        # ---- stages: a row per step of each distinct (component, axis, index)
+        depth = int(plane_stage_depth)
+        staged = {(po.component, po.axis, po.index): int(self.plane_re[q][0].numel()) for q, po in enumerate(planes)}
+        z_cells = sum(n for (_, axis, _), n in staged.items() if axis == 2)
+        if z_cells > 0 and depth > 64:
+            raise ValueError("plane_stage_depth must be at most 64")
+        self._stage_cells = sum(staged.values()) + prog.n_points  # what passes of several steps stage
+        self._stage_depth = min(64, max(4, depth // 4 * 4))
+        self.plane_stage = self._stage = None
+        self._add_workspace()
+        if z_cells > 0 and depth > 0:
+            shared = self._stage is not None and depth == self._stage_depth
+            self.plane_stage = self._stage if shared else torch.empty((depth, z_cells), dtype=torch.float32,
+                                                                      device=dev)
+            prog.plane_stage = nat.ptr(self.plane_stage)
+            prog.plane_stage_floats = self.plane_stage.numel()
+            prog.plane_stage_depth = depth
+
+    def _add_workspace(self):
+        """Scratch of passes that take several steps at once, where the library would
+        take this run's steps that way."""
+        self.workspace, self._scratch, self._scratch_used, self._dropped = None, [], False, False
+        if not self._multi:
+            return
+        work = nat.MwWorkspace()
+        work.term_steps = 2
+        sizes = {"line_history": 4 * int(self.program.aux.n_e), "stage": self._stage_depth * self._stage_cells}
+        psi = {q: self.psi[name].shape for q, name in enumerate(PSI_NAMES[:6])
+               if name in self.psi and self.psi[name].numel()}
+        work.stage_depth, work.stage_floats = self._stage_depth, sizes["stage"]
+        unread = nat.ptr(self._fields[0]["Ex"])  # asked for, not yet allocated
+        for name, n in sizes.items():
+            setattr(work, name, unread if n else None)
+        for q in psi:
+            work.psi_e_alt[q] = unread
+        self.workspace = work
+        if self.pass_plan()[0] == 0:
+            self.workspace = None
+            return
+
+        def scratch(shape):
+            self._scratch.append(torch.empty(shape, dtype=torch.float32, device=self.device))
+            return nat.ptr(self._scratch[-1])
+        for q, shape in psi.items():
+            work.psi_e_alt[q] = scratch(shape)
+        if sizes["line_history"]:
+            work.line_history = scratch(sizes["line_history"])
+        if sizes["stage"]:
+            work.stage = scratch((self._stage_depth, self._stage_cells))
+            self._stage = self._scratch[-1]
+
+    def drop_workspace(self):
+        """Give back the scratch that only this run's own passes use (a batch advances its
+        scenes without it); ``run`` makes it again."""
+        if self._scratch_used:  # perhaps still by a pass on another stream
+            torch.cuda.synchronize(self.device)
+        self.workspace, self._scratch, self._scratch_used, self._dropped = None, [], False, self.workspace is not None
+        self._stage = None
 
     @property
     def fields(self):
@@ -364,6 +391,9 @@ class DeviceRun:
         count = self.plan.time_steps - self.step_index if count is None else int(count)
         if count <= 0:
             return self
+        if self._dropped:
+            self._add_workspace()
+        self._scratch_used = self.workspace is not None
         with torch.cuda.device(self.device):
             rc = self.lib.mw_run_steps_ws(ctypes.byref(self.program),
                                           ctypes.byref(self.workspace) if self.workspace is not None else None,
