@@ -2,8 +2,7 @@
 float64 oracle where its tiles, chunks and stages end.
 
 Shapes are node counts around a tile's own 60 (two steps) and 62 (one step) columns and
-12 / 14 rows, the last one large enough that costlier tiles get shorter chunks of their
-own.  Runs are split so that single steps, pairs of two-step passes and stage blocks
+12 / 14 rows, all in equal blocks for passes of two steps.  Runs are split so that single steps, pairs of two-step passes and stage blocks
 begin at odd places.  Tolerance 1e-5 of a family's peak: about ten roundings of 2^-24
 per sample and step over 22 steps."""
 

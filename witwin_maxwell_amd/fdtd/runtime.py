@@ -47,12 +47,19 @@ class DeviceRun:
     double-buffered, one set of launches per step); ``fused=False`` the two-kernel
     in-place path.  Both handle every face mode, periodic included.
 
-    ``plane_stage_depth`` (0 = off): the samples of z-normal plane monitors are
+    ``plane_stage_depth``: the samples of z-normal plane monitors are
     copied into a stage of that many steps and added to their sums once per block
-    of steps, instead of the sums being read and written after every step.
+    of steps, instead of the sums being read and written after every step (0).
+    Passes that take two steps stage every observer, in that many rows (the multiple of
+    four below, at least four, also for 0).  The sums are the same to the bit.
 
     ``multi_step=False`` keeps every step a pass of its own, with the rounding of the
-    launches that capture and reverse steps for gradients."""
+    launches that capture and reverse steps for gradients.  It is also for a caller that
+    runs a step or two at a time on a small layered scene without z planes: passes of
+    two steps need four in a row, and a single step of the march takes up to a third more
+    than the separate launches there (63 x 74 x 166, CPML 16, an x flux plane: 52 us in
+    calls of one step against 40, and 34 against 40 in longer ones; with z planes, without
+    layers and from about 160^3 on single steps are the march's too)."""
 
     def __init__(self, plan: FDTDPlan, device="cuda", fused=None, plane_stage_depth=32, multi_step=True):
         self.plan = plan
