@@ -1727,9 +1727,9 @@ int mw_run_steps_ws(const mw_program* p, const mw_workspace* ws, int32_t first, 
     const int64_t off = (int64_t)from * p->nf_obs;
     if (zflush.count > 0) {
       zflush.stage = row;
-      hipLaunchKernelGGL(mw::flush_zstage_kernel, dim3(grid_blocks(zstage_cells), zflush.count), dim3(256), 0, s,
-                         zflush, rows, p->nf_obs, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off,
-                         p->obs_h_sin + off);
+      const auto kernel = rows <= 4 ? mw::flush_zstage_kernel<4> : mw::flush_zstage_kernel<mw::kMaxStageDepth>;
+      hipLaunchKernelGGL(kernel, dim3(grid_blocks(zstage_cells), zflush.count), dim3(256), 0, s, zflush, rows,
+                         p->nf_obs, p->obs_e_cos + off, p->obs_e_sin + off, p->obs_h_cos + off, p->obs_h_sin + off);
       if (int r = check_launch("flush_zstage")) return r;
     }
     if (march && p->n_points > 0) {

@@ -56,10 +56,11 @@ class DeviceRun:
     ``multi_step=False`` keeps every step a pass of its own, with the rounding of the
     launches that capture and reverse steps for gradients.  It is also for a caller that
     runs a step or two at a time on a small layered scene without z planes: passes of
-    two steps need four in a row, and a single step of the march takes up to a third more
-    than the separate launches there (63 x 74 x 166, CPML 16, an x flux plane: 52 us in
-    calls of one step against 40, and 34 against 40 in longer ones; with z planes, without
-    layers and from about 160^3 on single steps are the march's too)."""
+    two steps need four in a row, and a single step of the march takes up to a quarter more
+    than the separate launches there (63 x 74 x 166, CPML 16, an x flux plane: 46 us in
+    calls of one step against 40, and 34 against 40 in longer ones; 54 x 154 x 190 with
+    running sums 77 against 62, and 60 against 61).  With z planes, without layers and from
+    about 160^3 on single steps are the march's too."""
 
     def __init__(self, plan: FDTDPlan, device="cuda", fused=None, plane_stage_depth=32, multi_step=True):
         self.plan = plan
