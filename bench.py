@@ -491,7 +491,7 @@ def _short(name):
     if "__amd_rocclr_copyBuffer" in name:
         return "copy"
     for key in ("lean_step_kernel", "lean_batch_kernel", "zedge_step_kernel", "zedge_batch_kernel",
-                "zends_step_kernel"):
+                "zends_step_kernel", "march_kernel"):
         if key in name:
             return name[name.index(key):].split("(")[0]
     return name.split("(")[0][:80]
@@ -577,8 +577,8 @@ def summarize(argv):
             # the committed form that the forward workload reads back as roofline.traffic:
             # the step kernels' bytes per step, keyed by the tiling they were measured at
             calib = summary.pop("_calibration")
-            step = step_traffic(summary)
-            summary = {"by_tiling": {argv[3]: {STEP_KERNEL: step, "_per_kernel_bytes": summary,
+            label, step = step_traffic(summary)
+            summary = {"by_tiling": {argv[3]: {label: step, "_per_kernel_bytes": summary,
                                                "_calibration": calib}}}
         print(json.dumps(summary, indent=1))
     else:
@@ -593,9 +593,13 @@ _STEP_FAMILIES = ("lean_step_kernel", "shell_h_lean_kernel", "zends_step_kernel"
 
 
 def step_traffic(per_kernel):
-    """HBM bytes of one single-pass step: every kernel mw_run_steps launches for
-    the step itself (the monitors' gather/fold excluded, as in the step timing)."""
-    return sum(v["total_bytes"] for k, v in per_kernel.items() if any(f in k for f in _STEP_FAMILIES))
+    """(kernel label, HBM bytes) of one pass: a march's pass of two steps with its term
+    preparation, else every kernel mw_run_steps launches for a single-pass step itself
+    (the monitors' gather/fold excluded, as in the step timing)."""
+    march = [k for k in per_kernel if "march_kernel<2" in k or "march_prepare" in k]
+    if any("march_kernel" in k for k in march):
+        return MARCH_KERNEL, sum(per_kernel[k]["total_bytes"] for k in march)
+    return STEP_KERNEL, sum(v["total_bytes"] for k, v in per_kernel.items() if any(f in k for f in _STEP_FAMILIES))
 
 
 def _fastest(timings, n=6):

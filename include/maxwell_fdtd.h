@@ -254,8 +254,9 @@ typedef struct mw_program {
   const mw_term* e_terms;
   /* observers: weight tables are (total_steps, nf) float32 in device memory */
   int32_t nf_obs, n_planes, n_points;
-  /* single-pass tiling of the z ends: 0 or 2 = interior tiles aligned to the z
-   * PML slabs with the z ends in the per-cell shell, 1 = z-edge tiles beside the
+  /* single-pass tiling of the z ends: 0 = the library's choice (with a workspace,
+   * passes of two steps where they pay, see mw_pass_plan; else as 2), 2 = interior
+   * tiles aligned to the z PML slabs with the z ends in the per-cell shell, 1 = z-edge tiles beside the
    * interior tiles, 3 = interior tiles aligned as for 2 and both z ends of two
    * rows in one wavefront (when each end and a halo lane fit 32 lanes and the z
    * faces are not periodic; otherwise as 2), 4 = as 3 with the z-end launch on a

@@ -16,10 +16,12 @@
 // the halo: T rows, columns and planes at each side of a tile are computed again by the
 // neighbours (16 - 2T of 16 rows, 64 - 2T of 64 columns are a tile's own), whose loads
 // mostly hit L2 because the blocks resident on an XCD are neighbouring tiles marching
-// together.  What is left is the rate of a CU's vector memory instructions and the two
-// barriers a plane: per step, launches before -> march, PEC box of 257^3 344 -> 192 us,
-// 129^3 46 -> 32, 49^3 16 -> 8; with CPML on all faces 281^3
-// 527 -> 395 us, 185^3 172 -> 146, 105^3 42 -> 34, 49^3 24 -> 15.
+// together.  A pass over 281^3 nodes with CPML moves 2.22 GB of HBM at 2.4 TB/s (separate
+// launches 1.98 GB a step).  What is left is the rate of a CU's vector memory instructions
+// (324 a wavefront of sixteen planes, 43.7 thousand a CU and pass, 51 cycles each) and the
+// two barriers a plane; the wavefronts wait for half of their cycles.  us per step,
+// separate launches -> march: PEC box of 257^3 370 -> 184, 129^3 47 -> 32, 65^3 19 -> 13;
+// with CPML 12 and a plane wave 281^3 567 -> 424, 185^3 195 -> 174, 105^3 56 -> 45.
 //
 // Sixteen rows per block keep the share of halo rows low (4 of 16 at T = 2) and
 // fill a CU with one block (at most 128 VGPRs), so register use up to that costs no
@@ -154,7 +156,7 @@ __device__ __forceinline__ float scaled(float a, float b) {
   return a * b;
 }
 
-// The march's arguments where the launch (or a batch's table) keeps them.  `fresh`
+// The march's arguments where the launch keeps them.  `fresh`
 // hides where a pointer came from, so what is read through it is read there: the
 // arguments of the rarer work (layers, sums, terms) would otherwise all be hoisted
 // out of the plane loop and spilled, and cost every plane of every tile.

@@ -746,9 +746,9 @@ int march_tiles(int n, int width, int steps) {
 }
 
 // The march's blocks.  A block's plane takes as long as its wavefronts' loads and
-// stores (about 28 cycles of a CU each, whatever they carry: 15 of them a plane for
-// fields and coefficients cost 2.8 us on a full chip at 129^3, 23 with one axis of
-// CPML or with four observed components 4.3-4.6), so tiles are weighed by their count:
+// stores, whatever they carry (one more in every wavefront costs a plane 0.19-0.20 us
+// without layers and 0.20-0.27 us with CPML, over scenes of 97^3 to 225^3), so tiles are
+// weighed by their count, 15 for fields and coefficients, 8 for an axis of CPML:
 // z tiles by what lies in them, tile rows at the y ends by their layers, planes at the
 // x ends by theirs.  One block fills a CU, so the grid is cut until every CU has one:
 // the most costly block decides, and costlier tiles get more and shorter chunks.
