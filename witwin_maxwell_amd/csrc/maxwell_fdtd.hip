@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -896,31 +897,49 @@ int64_t march_blocks(const mw_program* p, const StageLayout& stage, int steps, m
   return hi;
 }
 
-// Do two-step passes, their busiest CU at `cost`, beat the separate launches of a
-// layered scene?  Both sides were measured on 118 scenes of CPML 8-12 from 105^3 to 281^3
-// nodes (cubes, slabs of 67-89 columns, rods), with a dipole or a plane wave, with and
-// without flux planes, lossless and lossy.  A march takes 0.115 us a step and unit of
-// cost (0.10-0.14), 1.5 times that where conductivity makes the coefficients general; the
-// separate launches 28 us a step, 23 us per million nodes (17-30) and 50 us per million samples
-// of z planes.  The side this picks is on average 0.5 % slower than the faster one, at
-// most 13 %.  us a step, march / separate: 201 x 101 x 67 with two z flux planes 90 / 71,
-// 161^3 127 / 149, 185^3 209 / 211, 225^3 278 / 324; 401 x 65 x 125 without planes 99 / 84;
-// lossy 201 x 101 x 67 86 / 64, 201^3 270 / 259, 121^3 66 / 75, 74^3 46 / 43.  Smaller
-// grids are left to the march (73^3 38 / 43), and so are scenes without layers (129^3 PEC
-// 32 / 47, lossy 47 / 55) and with running sums (121^3, one frequency, 58 / 89).
+// Do two-step passes beat the separate launches of a layered scene?  Both sides were
+// measured on 284 of them, CPML 6-12, 2048 to 33720 tile planes: 118 on a grid of shapes
+// (cubes, slabs, rods; with and without flux planes; lossless and lossy), 166 drawn at
+// random with boxes, vacuum or loss.  A march takes 0.115 us a step and unit of its busiest
+// CU's cost (0.09-0.14), 1.4 times that where conductivity makes the coefficients general.
+// The separate launches take 24 us a step, 9 more with time-shifted sources, 12 us per
+// million nodes of their interior tiles (63 columns, whole), 20 outside them, 55 us per
+// million samples of z planes, and 0.18 us per megabyte beyond the 250 that the last-level
+// cache keeps from step to step.  The march has the benefit of a ninth, since its errors are
+// the larger ones: 0.102.  The side this picks is on average 0.9 % slower than the faster
+// one, in 26 of the 284 by more than 3 %, at most 22 %.
+// us a step, march / separate: 201 x 101 x 67 with two z flux planes 90 / 71, 161^3 127 / 149,
+// 185^3 209 / 211, 225^3 278 / 324; 401 x 65 x 125 without planes 99 / 84; lossy 201 x 101 x 67
+// 86 / 64, 185^3 244 / 209, 121^3 66 / 75.  Smaller grids are left to the march (73^3 38 / 43)
+// unless lossy, which lose from 700 tile planes on (74^3 46 / 43, 75 x 316 x 59 65 / 59, 81 x
+// 116 x 100 56 / 48).  So are scenes without layers (129^3 PEC 32 / 47, lossy 47 / 55) and
+// with running sums (121^3, one frequency, 58 / 89).
 // `two` takes the blocks of a two-step pass where the answer needs them.
 bool march_pays(const mw_program* p, const StageLayout& stage, mw::MarchArgs* two) {
-  const int64_t tile_planes = (int64_t)march_tiles(p->grid.nz, mw::kMarchCols, 2) *
-                              march_tiles(p->grid.ny, mw::kMarchRows, 2) * p->grid.nx;
+  const mw_grid& g = p->grid;
+  const mw_cpml& c = p->cpml;
+  const int64_t tile_planes = (int64_t)march_tiles(g.nz, mw::kMarchCols, 2) *
+                              march_tiles(g.ny, mw::kMarchRows, 2) * g.nx;
   const bool general = coef_mode(p->coeffs) == 0;
-  if (!p->cpml.enabled || p->nf_dft > 0 || tile_planes < (general ? 700 : 2048)) return true;
-  const int64_t cost = march_blocks(p, stage, 2, two);
-  int64_t samples = 0;
+  if (!c.enabled || p->nf_dft > 0 || tile_planes < (general ? 700 : 2048)) return true;
+  if (tile_planes < 2048) return false;
+  const double march_ns = 102.0 * march_blocks(p, stage, 2, two) * (general ? 1.4 : 1.0);
+  const double n[3] = {(double)g.nx, (double)g.ny, (double)g.nz}, nodes = n[0] * n[1] * n[2];
+  double inner[3], bytes = 48.0 * nodes;
+  for (int a = 0; a < 3; ++a) {
+    const int q = a == 0 ? 2 : a - 1, layers = c.psi_low[q] + c.psi_high_len[q];  // an E-side psi of that axis
+    inner[a] = std::max(0.0, n[a] - layers);
+    bytes += 8.0 * 4 * layers * nodes / n[a];
+  }
+  for (int q = 0; q < 6; ++q) bytes += 4.0 * nodes * ((p->coeffs.decay[q] != nullptr) + (p->coeffs.curl[q] != nullptr));
+  bool shifted = false;
+  for (int i = 0; i < p->n_e_terms; ++i) shifted = shifted || p->e_terms[i].kind == MW_TERM_SHIFTED;
+  double samples = 0;
   for (int q = 0; q < stage.count; ++q)
     if (stage.planes[q].axis == 2) samples += stage.planes[q].cells;
-  const double nodes = (double)p->grid.nx * p->grid.ny * p->grid.nz;
-  const double march_ns = 115.0 * cost * (general ? 1.5 : 1.0);
-  return march_ns < 28e3 + 0.023 * nodes + 0.050 * samples;
+  return march_ns < 24e3 + (shifted ? 9e3 : 0.0) + 0.012 * inner[0] * inner[1] * 63.0 * std::ceil(inner[2] / 63.0) +
+                        0.020 * (nodes - inner[0] * inner[1] * inner[2]) + 0.055 * samples +
+                        0.00018 * std::max(0.0, bytes - 250e6);
 }
 
 // May the program's steps be taken by the march, one at a time (1) or two (2), or
