@@ -749,23 +749,28 @@ int march_tiles(int n, int width, int steps) {
 // The march's blocks.  A block's plane takes as long as its wavefronts' loads and
 // stores, whatever they carry (one more in every wavefront costs a plane 0.19-0.20 us
 // without layers and 0.20-0.27 us with CPML, over scenes of 97^3 to 225^3), so tiles are
-// weighed by their count, 15 for fields and coefficients, 8 for an axis of CPML:
+// weighed by their count, 15 for fields and coefficients, 8 for an axis of CPML, 1 for an
+// observed z plane, whose samples a few wavefronts store for all (with 2, 59 drawn scenes
+// took 4 % longer on average, 8 % from 8192 tile planes on; 201^3 with two flux planes 249
+// us a step against 204):
 // z tiles by what lies in them, tile rows at the y ends by their layers, planes at the
 // x ends by theirs.  One block fills a CU, so the grid is cut until every CU has one:
 // the most costly block decides, and costlier tiles get more and shorter chunks.
 // Small grids, where a plane takes its latency whatever lies in it, get equal blocks:
-// passes of two steps below 1536 tile planes (us a step of equal blocks / by weight, CPML,
-// two z flux planes: 73^3, 876 tile planes, 39 / 42; 89^3, 1424, 50 / 52; 105^3, 1890,
-// 58 / 51), passes of one below 600 (CPML 8, a dipole: 61 x 45 x 122, 488, 23.3 / 23.7;
-// 73^3 33.0 / 31.4; 85^3 37 / 32, with one z flux plane 44 / 37; 97^3 42 / 37).
-// Layered scenes beyond 20000 tile planes use blocks of sixteen planes: many short ones
-// even the load out by themselves, and keep the planes in use contiguous (CPML 12, a
-// plane wave, without and with two z flux planes, us a step of sixteen planes / by
-// weight: 241^3, 19280 tile planes, 330 / 273 and 338 / 303; 225 x 225 x 145, 12825, 211 /
-// 174 and 253 / 226; 185 x 265 x 265, 20350, 288 / 274 and 315 / 348; 281 x 185 x 281,
-// 22480, 296 / 340 and 324 / 346; 249^3, 26145, 351 / 389 and 378 / 402), and from 16384
-// on where the weighted blocks come out a tenth costlier (189 x 197 x 311, CPML 8, 235 /
-// 272, its costs 1982 and 2334; 2083 and 2007 for the 241^3 above).
+// passes of two steps below 1536 tile planes unless weighing saves a fifth of the costliest
+// of those (us a step of equal blocks / by weight, CPML 10, a plane wave, none and two z
+// flux planes: 61 x 45 x 121, saves 0.07, 24.4 / 28.3 and 28.6 / 32.3; 117 x 49 x 77, 0.12
+// and 0.19, 32.7 / 34.1 and 38.1 / 38.6; 65^3, 0.21 and 0.27, 32.5 / 28.2 and 38.3 / 35.9; 89^3,
+// 0.17 and 0.24, 40.4 / 38.5 and 47.8 / 44.1; with a dipole and CPML 6-8 two scenes that save
+// 0.17 lost 14 %), passes of one below 600 (CPML 8, a dipole: 61 x 45 x 122,
+// 488, 23.3 / 23.7; 73^3 33.0 / 31.4; 85^3 37 / 32; 97^3 42 / 37).
+// Layered scenes from 16384 tile planes on use blocks of sixteen planes where those come
+// out cheaper or no list fits: many short ones even the load out by themselves, and keep
+// the planes in use contiguous (CPML 12, a plane wave, none and two z flux planes, costs
+// and us a step of sixteen planes / by weight: 225^3 1858 / 1848, 317 / 251 and 2112 / 2159,
+// 324 / 227; 281 x 185 x 281 2324 / 2704, 295 / 335 and 2589 / 2704, 324 / 342; 185 x 265 x 265
+// 2097 / 2320, 288 / 270 and 2338 / 2320, 316 / 281; 249^3, which no list of 256 fits, 350 and
+// 379, in rounds of equal blocks 387 and 400).
 // Returns the cost of the busiest CU, in those counts.
 int64_t march_blocks(const mw_program* p, const StageLayout& stage, int steps, mw::MarchArgs* out) {
   mw::MarchArgs& a = *out;
@@ -788,7 +793,7 @@ int64_t march_blocks(const mw_program* p, const StageLayout& stage, int steps, m
     const int k0 = z * own_z, k1 = std::min(g.nz, k0 + mw::kMarchCols);
     int cost = kPlain + (k0 < low(2) || k1 > high(2, g.nz) ? kLayer : 0);
     for (int q = 0; q < stage.count; ++q)
-      if (stage.planes[q].axis == 2 && stage.planes[q].index >= k0 && stage.planes[q].index < k1) cost += steps;
+      if (stage.planes[q].axis == 2 && stage.planes[q].index >= k0 && stage.planes[q].index < k1) cost += 1;
     for (int f = 0; f < 2; ++f)
       for (int i = 0; i < (f ? p->n_e_terms : p->n_h_terms); ++i) {
         const mw_term& t = f ? p->e_terms[i] : p->h_terms[i];
@@ -810,13 +815,13 @@ int64_t march_blocks(const mw_program* p, const StageLayout& stage, int steps, m
     return all / mw::kMarchBlocks;
   };
   if (p->xchunk > 0) return even(p->xchunk);
-  if (c.enabled && (int64_t)tiles * g.nx >= 20000) return even(16);
   int cost_z[mw::kMarchBlocks], cost_y[mw::kMarchBlocks];
   struct Kind {  // tiles of one cost: how many, and where the first one's blocks are listed
     int plane, count, first, blocks;
   } kinds[mw::kMarchBlocks];
   int n_kinds = 0;
-  bool alike = (int64_t)tiles * g.nx < (steps == 2 ? 1536 : 600);
+  const int64_t tile_planes = (int64_t)tiles * g.nx;
+  bool alike = steps == 1 && tile_planes < 600;
   if (tiles <= mw::kMarchBlocks) {
     bool same = layers == 0;
     for (int z = 0; z < a.tiles_z; ++z) cost_z[z] = tile_cost(z);
@@ -846,25 +851,37 @@ int64_t march_blocks(const mw_program* p, const StageLayout& stage, int steps, m
     return n;
   };
   int lo = 0, hi = (g.nx + extra) * (kPlain + 64) + layers * kLayer + 64 * MW_MAX_TERMS;
-  if (alike || tiles > mw::kMarchBlocks || g.nx > 65535 || total(hi) > mw::kMarchBlocks) {  // whole rounds of equal blocks
-    int best = std::min(g.nx, mw::kMarchPlanes);
-    int64_t cost = INT64_MAX;
+  // whole rounds of equal blocks: their planes, and the cost of the costliest tile's rounds
+  auto rounds = [&](int* chunk) {
+    int64_t planes = INT64_MAX;
     for (int n = (g.nx + mw::kMarchPlanes - 1) / mw::kMarchPlanes; n <= g.nx; ++n) {
-      const int chunk = (g.nx + n - 1) / n;
-      const int64_t per_xcd = ((int64_t)tiles * ((g.nx + chunk - 1) / chunk) + 7) / 8;
-      const int64_t t = ((per_xcd + 31) / 32) * (chunk + extra);
-      if (t < cost) {
-        cost = t;
-        best = chunk;
+      const int cut = (g.nx + n - 1) / n;
+      const int64_t per_xcd = ((int64_t)tiles * ((g.nx + cut - 1) / cut) + 7) / 8;
+      const int64_t t = ((per_xcd + 31) / 32) * (cut + extra);
+      if (t < planes) {
+        planes = t;
+        *chunk = cut;
       }
     }
-    return even(best);
+    return planes;
+  };
+  int chunk = std::min(g.nx, mw::kMarchPlanes);
+  if (alike || tiles > mw::kMarchBlocks || g.nx > 65535 || total(hi) > mw::kMarchBlocks) {
+    if (c.enabled && !alike && tile_planes >= 16384) return even(16);
+    rounds(&chunk);
+    return even(chunk);
   }
   while (hi - lo > 1) {
     const int mid = (lo + hi) / 2;
     (total(mid) <= mw::kMarchBlocks ? hi : lo) = mid;
   }
-  if (c.enabled && (int64_t)tiles * g.nx >= 16384 && 10 * hi > 11 * even(16)) return even(16);
+  if (c.enabled && tile_planes >= 16384 && 100 * (int64_t)hi > 103 * even(16)) return even(16);
+  if (steps == 2 && tile_planes < 1536) {
+    int most = 0;  // the costliest tile, of which a block has at least one plane
+    for (int q = 0; q < n_kinds; ++q) most = std::max(most, kinds[q].plane);
+    hi = std::max(hi, (1 + extra) * most);
+    if (5 * (int64_t)hi > 4 * rounds(&chunk) * most) return even(chunk);
+  }
   a.chunk = 0;
   a.blocks = 0;
   for (int y = 0; y < a.tiles_y; ++y)
@@ -898,22 +915,21 @@ int64_t march_blocks(const mw_program* p, const StageLayout& stage, int steps, m
 }
 
 // Do two-step passes beat the separate launches of a layered scene?  Both sides were
-// measured on 284 of them, CPML 6-12, 2048 to 33720 tile planes: 118 on a grid of shapes
-// (cubes, slabs, rods; with and without flux planes; lossless and lossy), 166 drawn at
-// random with boxes, vacuum or loss.  A march takes 0.115 us a step and unit of its busiest
-// CU's cost (0.09-0.14), 1.4 times that where conductivity makes the coefficients general.
-// The separate launches take 24 us a step, 9 more with time-shifted sources, 12 us per
-// million nodes of their interior tiles (63 columns, whole), 20 outside them, 55 us per
-// million samples of z planes, and 0.18 us per megabyte beyond the 250 that the last-level
-// cache keeps from step to step.  The march has the benefit of a ninth, since its errors are
-// the larger ones: 0.102.  The side this picks is on average 0.9 % slower than the faster
-// one, in 26 of the 284 by more than 3 %, at most 22 %.
-// us a step, march / separate: 201 x 101 x 67 with two z flux planes 90 / 71, 161^3 127 / 149,
-// 185^3 209 / 211, 225^3 278 / 324; 401 x 65 x 125 without planes 99 / 84; lossy 201 x 101 x 67
-// 86 / 64, 185^3 244 / 209, 121^3 66 / 75.  Smaller grids are left to the march (73^3 38 / 43)
-// unless lossy, which lose from 700 tile planes on (74^3 46 / 43, 75 x 316 x 59 65 / 59, 81 x
-// 116 x 100 56 / 48).  So are scenes without layers (129^3 PEC 32 / 47, lossy 47 / 55) and
-// with running sums (121^3, one frequency, 58 / 89).
+// measured on 236 scenes of 2048 to 28912 tile planes drawn at random: CPML 6-12, boxes,
+// vacuum or loss, a dipole or a plane wave, flux planes or a point.  A march takes 0.115 us a
+// step and unit of its busiest CU's cost (0.10-0.14), 1.4 times that where conductivity
+// makes the coefficients general.  The separate launches take 28 us a step, 9 more with
+// time-shifted sources, 14 us per million nodes of their interior tiles (63 columns, whole),
+// 20 outside them, 35 us per million samples of z planes, and 0.18 us per megabyte beyond the
+// 250 that the last-level cache keeps from step to step.  The march has the benefit of a
+// twelfth, since its errors are the larger ones: 0.106.  The side this picks is on average 0.8 %
+// slower than the faster one, in 16 of the 236 by more than 3 %, at most 26 %; 0.88 of the
+// separate launches' time.  us a step, march / separate: 161^3 with two z flux planes 108 /
+// 148, 185^3 187 / 210, 225^3 227 / 324, 201 x 101 x 67 72 / 70; 401 x 65 x 125, CPML 8, 118 / 95,
+// without planes 98 / 84; lossy 201 x 101 x 67 86 / 64, 185^3 244 / 209, 121^3 64 / 73.  Smaller
+// grids are left to the march (73^3 38 / 43) unless lossy, which lose from 700 tile planes on
+// (74^3 46 / 43, 75 x 316 x 59 65 / 59, 81 x 116 x 100 56 / 48).  So are scenes without layers
+// (129^3 PEC 32 / 47, lossy 47 / 55) and with running sums (121^3, one frequency, 57 / 88).
 // `two` takes the blocks of a two-step pass where the answer needs them.
 bool march_pays(const mw_program* p, const StageLayout& stage, mw::MarchArgs* two) {
   const mw_grid& g = p->grid;
@@ -923,7 +939,7 @@ bool march_pays(const mw_program* p, const StageLayout& stage, mw::MarchArgs* tw
   const bool general = coef_mode(p->coeffs) == 0;
   if (!c.enabled || p->nf_dft > 0 || tile_planes < (general ? 700 : 2048)) return true;
   if (tile_planes < 2048) return false;
-  const double march_ns = 102.0 * march_blocks(p, stage, 2, two) * (general ? 1.4 : 1.0);
+  const double march_ns = 106.0 * march_blocks(p, stage, 2, two) * (general ? 1.4 : 1.0);
   const double n[3] = {(double)g.nx, (double)g.ny, (double)g.nz}, nodes = n[0] * n[1] * n[2];
   double inner[3], bytes = 48.0 * nodes;
   for (int a = 0; a < 3; ++a) {
@@ -937,8 +953,8 @@ bool march_pays(const mw_program* p, const StageLayout& stage, mw::MarchArgs* tw
   double samples = 0;
   for (int q = 0; q < stage.count; ++q)
     if (stage.planes[q].axis == 2) samples += stage.planes[q].cells;
-  return march_ns < 24e3 + (shifted ? 9e3 : 0.0) + 0.012 * inner[0] * inner[1] * 63.0 * std::ceil(inner[2] / 63.0) +
-                        0.020 * (nodes - inner[0] * inner[1] * inner[2]) + 0.055 * samples +
+  return march_ns < 28e3 + (shifted ? 9e3 : 0.0) + 0.014 * inner[0] * inner[1] * 63.0 * std::ceil(inner[2] / 63.0) +
+                        0.020 * (nodes - inner[0] * inner[1] * inner[2]) + 0.035 * samples +
                         0.00018 * std::max(0.0, bytes - 250e6);
 }
 
